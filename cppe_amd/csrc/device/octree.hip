@@ -428,19 +428,23 @@ void build_octree(System& S, const double* pos) {
 // Dual-tree traversal (fmm/calculate.cc:74-127), one generation of the frontier per launch. A
 // generation reads its length from the counters, so the generations follow each other without the
 // host: a pair splits one of its cells per generation, 2 max_level + 1 of them empty the frontier.
+// A list that is full is reported in the generation's own word, and a generation looks only at the word of the one
+// before it, which no launch still writes: every wavefront of a block takes the same way to the barriers. (A word that
+// other blocks set meanwhile let some wavefronts of a block leave, the rest then counted LDS nobody had written.)
 // Slots are taken once per block, list and kTravTile pairs (classify, block prefix sums, one atomic per
 // list, classify again and write): atomics on one address complete one after another, and a slot per pair
 // or per wavefront made the traversal the longest set-up kernel (0.84 ms at 120,000 sites, 7.6 ms at
 // 300,000; now 0.16 ms and 0.57 ms).
 // ---------------------------------------------------------------------------------------------
 constexpr int kTravGen = 2 * kMaxLevel + 1;
-enum TravCount { TC_M2L = 0, TC_P2P, TC_OVER, TC_FRONT, TC_COUNT = TC_FRONT + kTravGen + 1 };
+enum TravCount { TC_M2L = 0, TC_P2P, TC_FRONT, TC_OVER = TC_FRONT + kTravGen + 1, TC_COUNT = TC_OVER + kTravGen + 1 };
 struct TravOut {
   int2* next;
   unsigned long long* m2l;  // (target << 32) | source
   unsigned long long* p2p;  // (target << 32) | source
-  int* counters;            // TravCount: list lengths, overflow flag, frontier length per generation
-  int cap_next, cap_m2l, cap_p2p;
+  // TravCount: list lengths; per generation the frontier's length, and whether a list was full before it
+  unsigned long long* counters;
+  long long cap_next, cap_m2l, cap_p2p;
 };
 
 struct TravCells {
@@ -468,9 +472,14 @@ __device__ __forceinline__ int trav_kind(const TravCells& c, int A, int B, int& 
 
 constexpr int kTravPer = 8, kTravTile = 256 * kTravPer;
 __global__ __launch_bounds__(256) void k_traverse(int gen, const int2* __restrict__ front, TravOut o, TravCells c) {
-  __shared__ int part[3][4], base[3];
-  if (o.counters[TC_OVER]) return;
-  const int nfront = o.counters[TC_FRONT + gen], tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  __shared__ int part[3][4];
+  __shared__ long long base[3];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  if (o.counters[TC_OVER + gen]) {  // (final since the last launch: uniform over the grid)
+    if (blockIdx.x == 0 && tid == 0) o.counters[TC_OVER + gen + 1] = 1;
+    return;
+  }
+  const long long nfront = o.counters[TC_FRONT + gen];  // (within the capacity, else the word above is set)
   for (long long t0 = (long long)blockIdx.x * kTravTile; t0 < nfront; t0 += (long long)gridDim.x * kTravTile) {
     // (thread tid takes the pairs t0 + tid + 256 q: coalesced reads; the lists are sorted afterwards)
     int num[3] = {0, 0, 0}, k, c0;
@@ -483,7 +492,7 @@ __global__ __launch_bounds__(256) void k_traverse(int gen, const int2* __restric
       num[1] += kd == 1;
       num[2] += k;
     }
-    int at[3];
+    long long at[3];
     __syncthreads();  // (the previous tile's reads of part and base are done)
 #pragma unroll
     for (int l = 0; l < 3; ++l) {
@@ -494,8 +503,8 @@ __global__ __launch_bounds__(256) void k_traverse(int gen, const int2* __restric
     __syncthreads();
     if (tid < 3) {
       const int total = part[tid][0] + part[tid][1] + part[tid][2] + part[tid][3];
-      int* counter    = &o.counters[tid == 0 ? TC_M2L : tid == 1 ? TC_P2P : TC_FRONT + gen + 1];
-      base[tid]       = total ? atomicAdd(counter, total) : 0;
+      unsigned long long* counter = &o.counters[tid == 0 ? TC_M2L : tid == 1 ? TC_P2P : TC_FRONT + gen + 1];
+      base[tid] = total ? (long long)atomicAdd(counter, (unsigned long long)total) : 0;
     }
     __syncthreads();
 #pragma unroll
@@ -503,11 +512,11 @@ __global__ __launch_bounds__(256) void k_traverse(int gen, const int2* __restric
       at[l] += base[l];
       for (int w = 0; w < wv; ++w) at[l] += part[l][w];
     }
-    const int cap[3] = {o.cap_m2l, o.cap_p2p, o.cap_next};
+    const long long cap[3] = {o.cap_m2l, o.cap_p2p, o.cap_next};
 #pragma unroll
     for (int l = 0; l < 3; ++l)
       if (num[l] && at[l] + num[l] > cap[l]) {
-        atomicExch(&o.counters[TC_OVER], 1);
+        atomicExch(&o.counters[TC_OVER + gen + 1], 1ull);
         num[0] = num[1] = num[2] = -1;
       }
     if (num[0] < 0) continue;  // (no barrier before the next tile's first)
@@ -956,7 +965,7 @@ void build_lists(System& S) {
   long long cap_m2l  = 512ll * T.ncells + 4096;
   long long cap_p2p  = 256ll * T.nleaves + 4096;
   long long cap_next = std::max<long long>(cap_m2l, T.level_offset[1]);
-  dbuf<int> counters;
+  dbuf<unsigned long long> counters;
   counters.alloc(TC_COUNT);
   for (int attempt = 0; attempt < 6; ++attempt) {
     dbuf<int2> fa, fb;
@@ -970,19 +979,19 @@ void build_lists(System& S) {
     std::vector<int2> seed(nroots);
     for (int c = 0; c < nroots; ++c) seed[c] = make_int2(c, c);
     CPPE_HIP_CHECK(hipMemcpyAsync(fa.p, seed.data(), sizeof(int2) * nroots, hipMemcpyHostToDevice, st));
-    int h_cnt[TC_COUNT] = {};
-    h_cnt[TC_FRONT]     = nroots;
+    unsigned long long h_cnt[TC_COUNT] = {};
+    h_cnt[TC_FRONT]                    = nroots;
     CPPE_HIP_CHECK(hipMemcpyAsync(counters.p, h_cnt, sizeof(h_cnt), hipMemcpyHostToDevice, st));
     const dim3 grid(std::min(2048, ceil_div(cap_next, kTravTile)));
     const TravCells cells{T.cx.p, T.cy.p, T.cz.p, T.crmax.p, T.nchild.p, T.child_first.p, theta};
     const int ngen = 2 * T.max_level + 1;
     for (int g = 0; g < ngen; ++g) {
-      TravOut o{g % 2 ? fa.p : fb.p, m2l.p, p2p.p, counters.p, (int)cap_next, (int)cap_m2l, (int)cap_p2p};
+      TravOut o{g % 2 ? fa.p : fb.p, m2l.p, p2p.p, counters.p, cap_next, cap_m2l, cap_p2p};
       hipLaunchKernelGGL(k_traverse, grid, dim3(256), 0, st, g, g % 2 ? fb.p : fa.p, o, cells);
     }
     CPPE_HIP_CHECK(hipMemcpyAsync(h_cnt, counters.p, sizeof(h_cnt), hipMemcpyDeviceToHost, st));
     CPPE_HIP_CHECK(hipStreamSynchronize(st));
-    const bool overflow = h_cnt[TC_OVER] != 0;
+    const bool overflow = h_cnt[TC_OVER + ngen] != 0;
     if (!overflow && h_cnt[TC_FRONT + ngen] != 0) throw std::runtime_error("octree: the traversal did not end");
     if (overflow) {
       cap_m2l *= 2;
@@ -990,8 +999,10 @@ void build_lists(System& S) {
       cap_next *= 2;
       continue;
     }
-    T.n_m2l = h_cnt[TC_M2L];
-    T.n_p2p = h_cnt[TC_P2P];
+    T.n_m2l = (long long)h_cnt[TC_M2L];
+    T.n_p2p = (long long)h_cnt[TC_P2P];
+    if (T.n_m2l > INT_MAX || T.n_p2p > INT_MAX)
+      throw std::runtime_error("octree: more interaction pairs than a 32-bit index addresses");
     dbuf<char> tmp;
     sort_keys(m2l, T.n_m2l, T.ncells, st, tmp);
     sort_keys(p2p, T.n_p2p, T.ncells, st, tmp);
