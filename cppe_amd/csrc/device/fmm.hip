@@ -36,7 +36,7 @@ CPPE_EXTERN_FMM(8)
 constexpr int kOverlapSites = 1536;
 // Launch shapes of a system that is neither tuned nor given a choice (cppe_hip_autotune /
 // cppe_hip_set_tune): what a program that only builds a system and solves runs with.
-static FmmTune default_tune(const System& S) {
+static FmmTune default_tune(System& S) {
   FmmTune t;
   const Octree& T = S.tree;
   t.near_block[0] = t.near_block[1] = 128;
@@ -58,10 +58,12 @@ static FmmTune default_tune(const System& S) {
   // FP64: chunks of 4; the symmetric form for the plain form's solves of larger systems with small
   // leaves, where sharing a pair's geometry outweighs the reverse blocks (a mixed solve runs one or
   // two FP64 applies, which would not pay for its lists). Its reverse slots are 32-bit indices: at
-  // most 3 values per site pair of different leaves, each unordered pair once.
+  // most 3 values per site pair of different leaves, each unordered pair once. It needs near lists that
+  // are symmetric, which those of a theta near 1 are not.
   const bool plain  = S.opts.precision == CPPE_HIP_PREC_FP64;
   const bool fits   = 1.5 * (double)T.p2p_site_pairs < 2147483647.0;
-  const bool sym    = plain && fits && S.n >= kSymTreeSites && S.n < (long long)kSymLeafSites * T.nleaves;
+  const bool sym    = plain && fits && S.n >= kSymTreeSites && S.n < (long long)kSymLeafSites * T.nleaves &&
+                   S.has_alpha && near_lists_symmetric(S);
   t.near_variant[0] = sym ? 9 : 7;
   t.near_block[0]   = sym ? 128 : 256;
   t.m2l_group[0] = t.m2l_group[1] = T.ncells < kM2lWideCells ? 64 : 16;
@@ -368,8 +370,9 @@ bool decode_overlap(int code, int& form, int& splits) {
 }
 
 void fmm_autotune(System& S, int reps, int* choice, double* ms) {
+  FmmState& F = state(S);
+  F.tune      = default_tune(S);  // (an earlier choice may be one that this tree does not allow)
   fmm_reserve(S, true, 1);
-  FmmState& F    = *S.fmm;
   hipStream_t st = S.stream;
   hipEvent_t ev[8];
   for (auto& e : ev) CPPE_HIP_CHECK(hipEventCreate(&e));
@@ -407,7 +410,8 @@ void fmm_autotune(System& S, int reps, int* choice, double* ms) {
       F.tune.overlap[prec] = 0;
       int best        = 0;
       for (int c = 0; c < kNNear; ++c) {
-        if (!near_variant_allowed(S, kNearCand[c][0])) {
+        if (!near_variant_allowed(S, kNearCand[c][0]) ||
+            (near_sym_variant(kNearCand[c][0]) && !near_lists_symmetric(S))) {
           m[c] = 0.0;  // not timed
           continue;
         }

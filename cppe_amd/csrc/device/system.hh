@@ -52,6 +52,7 @@ struct Octree {
   dbuf<long long> xsplit[2];
   double xdamp = 0.0;  // damping factor of the classification (valid for kernels with damping >= xdamp)
   SymLists sym[2][5];  // symmetric near field (FP64, FP32) with chunks of 4, 6, 8, 12, 16 targets (sym_slot)
+  int near_symmetric = -1;  // near_lists_symmetric's answer (-1: not asked yet)
   bool built = false;
 };
 
@@ -216,6 +217,7 @@ void build_octree(System& S, const double* pos);
 void device_scan(System& S, const int* in, int* out, int n);
 void build_lists(System& S);
 void build_near_expanded(System& S);
+bool near_lists_symmetric(System& S);
 // lists of the symmetric near-field kernel with chunks of ts targets (4, 6, 8, 12 or 16) into
 // S.tree.sym[prec][sym_slot(ts)] (prec: 0 FP64, 1 FP32)
 inline int sym_slot(int ts) { return ts <= 4 ? 0 : ts <= 6 ? 1 : ts <= 8 ? 2 : ts <= 12 ? 3 : 4; }

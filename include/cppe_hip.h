@@ -261,7 +261,8 @@ int cppe_hip_last_solve_info(cppe_hip_system* sys, int* info);
  *      leaves with a higher index, lanes = sources; the field at those sources goes to per-leaf
  *      reverse blocks that a gather pass adds in a fixed order (with the L2P term); block
  *      64/128/256. Single-right-hand-side B applies only: the system's other near-field launches
- *      then use variant 8.
+ *      then use variant 8. Needs symmetric near lists (a theta near 1 can leave pairs near from
+ *      one side only): not timed on other trees, and an error there when chosen by set_tune.
  * Then, for a staged or symmetric near variant (5-11), the whole apply is timed with the far field (P2M, M2M,
  * M2L, L2L) in series, on a second stream beside the near field (joined before an L2P pass; enqueued
  * after the near field or ahead of it), and with only M2L / L2L beside the near field after the
