@@ -139,7 +139,7 @@ void fmm_reserve_multi(System& S, bool mixed) {
     ensure_m2l_rec(S, S.stream);
   }
   ensure_pos4(S);
-  ensure_excl_near(S);
+  build_pair_skips(S);
   for (int prec = 0; prec <= (mixed ? 1 : 0); ++prec) {
     const int v = F.tune.near_variant[prec];
     if (v < 5) continue;
@@ -284,7 +284,7 @@ void fmm_reserve(System& S, bool mixed, int nrhs) {
   ensure_buf(F.L64, nc * fmm_lsize(0, p));
   ensure_buf(F.mu4, S.n);
   ensure_pos4(S);
-  ensure_excl_near(S);
+  build_pair_skips(S);
   if (mixed) {
     ensure_buf(F.M32, fmm_mbuf_size(nc, 0, p));
     ensure_buf(F.L32, nc * fmm_lsize(0, p));

@@ -82,9 +82,6 @@ struct FmmState {
   dbuf<double> Mc, Lc;    // combined kind (static fields, m = 0 / 2)
   dbuf<double> src10;     // staging of combined sources
   dbuf<double4> pos4;     // near-field source records: x, y, z, alpha_iso^(-1/6)
-  // per site, the exclusion partners whose pairs the near field adds (CSR, built once per tree)
-  dbuf<int> xn_off, xn_idx;
-  bool xn_built = false;
   int reserved_for[2] = {-1, -1};  // near variants (FP64, FP32) fmm_reserve last prepared for
   dbuf<double4> mu4;      // near-field dipole records (FP64 form)
   dbuf<float4> mu4f;      // near-field dipole records (FP32 form)
@@ -984,28 +981,26 @@ struct alignas(K == 1 ? 4 * sizeof(R) : 16) StagedRec {  // K = 1: two 16-byte (
   R m[3 * K];
 };
 
-// Geometry of one near-field pair of the staged kernel and of the exclusion pass (identical
-// arithmetic, so an excluded pair is taken out exactly as it was added). B2: the branch-free FP32
-// form for systems whose sites are all damped; di then carries the factor log2(e).
-// FAR: a source past the precision's far class for every target of the leaf (never the target
-// itself): the undamped geometry (FP32: from v >= 18 on, where the screening it leaves out moves
-// the field by less than the FP32 rounding; FP64 takes no far stages).
-template <typename R, bool DAMP, bool B2, bool FAR = false>
-__device__ __forceinline__ void staged_geo(R dx, R dy, R dz, R a, R& c3, R& cf) {
+// Geometry of one near-field pair. B2: the branch-free FP32 form for systems whose sites are all damped;
+// a then carries the factor log2(e). FAR: a source past the precision's far class for every target of the leaf (never
+// the target itself or a skipped pair): the undamped geometry (FP32: from v >= 18 on, where the screening it
+// leaves out moves the field by less than the FP32 rounding; FP64: from v >= 40 on, where it is exactly 1).
+// SELF0: a pair without displacement (the site itself, where the kernel takes it in) is zero; skip: this pair is.
+template <typename R, bool DAMP, bool B2, bool FAR, bool SELF0>
+__device__ __forceinline__ void staged_geo(R dx, R dy, R dz, R a, R& c3, R& cf, bool skip = false) {
   if constexpr (sizeof(R) == 8)
-    geo_m1_f64<DAMP && !FAR, !FAR>(dx, dy, dz, a, c3, cf);
+    geo_m1_f64<DAMP && !FAR, SELF0 && !FAR>(dx, dy, dz, a, c3, cf, skip);
   else if constexpr (FAR)
     geo_m1_f32<false, false>(dx, dy, dz, a, c3, cf);
   else if constexpr (B2)
-    geo_m1_f32_b2(dx, dy, dz, a, c3, cf);
+    geo_m1_f32_b2<SELF0>(dx, dy, dz, a, c3, cf, skip);
   else
-    geo_m1_f32<DAMP, true>(dx, dy, dz, a, c3, cf);
+    geo_m1_f32<DAMP, SELF0>(dx, dy, dz, a, c3, cf, skip);
 }
 
-// one pair against the K dipoles of a staged record; f holds 3 K accumulators
-template <typename R, bool DAMP, bool B2, int K, bool FAR = false>
-__device__ __forceinline__ void staged_pair(R xi, R yi, R zi, R di, const StagedRec<R, K>& r, R* f) {
-  const R dx = xi - r.x, dy = yi - r.y, dz = zi - r.z;
+// one pair against the K dipoles of a staged record, given its displacement; f holds 3 K accumulators
+template <typename R, bool DAMP, bool B2, int K, bool FAR = false, bool SELF0 = true>
+__device__ __forceinline__ void staged_pair(R dx, R dy, R dz, R di, const StagedRec<R, K>& r, R* f, bool skip = false) {
   if constexpr (FAR && sizeof(R) == 4) {
     float ri3, m3;
     geo_far_f32(dx, dy, dz, ri3, m3);
@@ -1015,7 +1010,7 @@ __device__ __forceinline__ void staged_pair(R xi, R yi, R zi, R di, const Staged
                   f[3 * k + 2]);
   } else {
     R c3, cf;
-    staged_geo<R, DAMP, B2, FAR>(dx, dy, dz, di * r.s, c3, cf);
+    staged_geo<R, DAMP, B2, FAR, SELF0>(dx, dy, dz, di * r.s, c3, cf, skip);
 #pragma unroll
     for (int k = 0; k < K; ++k)
       acc_m1(c3, cf, dx, dy, dz, r.m[3 * k], r.m[3 * k + 1], r.m[3 * k + 2], f[3 * k], f[3 * k + 1], f[3 * k + 2]);
@@ -1107,12 +1102,14 @@ __global__ __launch_bounds__(256) void k_fmm_near_st(NearArgs a, const int2* __r
       if (lane < q1 - q0 - 128) jnn = xsrc[q0 + 128 + lane];  // stage s + 2: its source index
     }
     // every pair of the near list, the self pair contributing zero; excluded near pairs are
-    // taken out afterwards by k_fmm_excl_sub with the same arithmetic
+    // taken out afterwards by k_fmm_skip_fix with the same arithmetic
     if (act) {
       if (DAMP && sizeof(R) == 4 && q0 >= qf) {  // far stage (uniform): undamped pairs, branch-free
-        for (int u = sl; u < cn; u += S) staged_pair<R, DAMP, B2, 1, true>(xi, yi, zi, di, sr[u], f);
+        for (int u = sl; u < cn; u += S)
+          staged_pair<R, DAMP, B2, 1, true>(xi - sr[u].x, yi - sr[u].y, zi - sr[u].z, di, sr[u], f);
       } else {
-        for (int u = sl; u < cn; u += S) staged_pair<R, DAMP, B2, 1>(xi, yi, zi, di, sr[u], f);
+        for (int u = sl; u < cn; u += S)
+          staged_pair<R, DAMP, B2, 1>(xi - sr[u].x, yi - sr[u].y, zi - sr[u].z, di, sr[u], f);
       }
     }
     wave_lds_barrier();
@@ -1314,16 +1311,10 @@ __global__ void k_pack_mu4(int n, const double* __restrict__ mu, MU4* __restrict
   out[i] = v;
 }
 
-// Whether exclusion partner k of site i is a pair the near field adds: a valid index other than
-// i, its first occurrence in i's list, and its leaf in the near list of i's leaf A (o0, o1: A's
-// list, sorted by source leaf; otherwise a far-field pair, which stays in).
-__device__ __forceinline__ bool excl_in_near(const NearArgs& a, int i, int k0, int k, int o0, int o1) {
-  const int e = a.eidx[k];
-  if (e < 0 || e >= a.n || e == i) return false;
-  for (int q = k0; q < k; ++q)
-    if (a.eidx[q] == e) return false;
-  const int B = a.leaf_of[e];
-  int lo = o0, hi = o1;
+// Whether leaf B is in the near list of leaf A.
+__device__ __forceinline__ bool leaves_near(const NearArgs& a, int A, int B) {
+  int lo = a.p2p_off[A], hi = a.p2p_off[A + 1];
+  const int end = hi;
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
     if (a.p2p_src[mid] < B)
@@ -1331,93 +1322,98 @@ __device__ __forceinline__ bool excl_in_near(const NearArgs& a, int i, int k0, i
     else
       hi = mid;
   }
-  return lo < o1 && a.p2p_src[lo] == B;
+  return lo < end && a.p2p_src[lo] == B;
 }
 
-// The partners excl_in_near accepts, per site in list order: their number into out[i] (off
-// null), or the partners themselves into out[off[i] ...].
-static __global__ __launch_bounds__(256) void k_excl_near(NearArgs a, const int* __restrict__ off,
-                                                         int* __restrict__ out) {
+// The pairs of a skip list that a near-field pass has treated otherwise than the field at the list's site wants
+// (pairs outside the near lists belong to the far field and stay). KEEP false, after the staged form (variants 5
+// and 6), which adds every pair: the pairs the site excludes are taken out, with that form's arithmetic. KEEP true,
+// after the symmetric forms, which skip a pair that either side excludes: those only the partner excludes are added.
+template <typename R, bool DAMP, bool B2, bool KEEP, typename MU4>
+__global__ __launch_bounds__(256) void k_fmm_skip_fix(NearArgs a, SkipLists sk, const MU4* __restrict__ mu4) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.n) return;
-  const int k0 = a.eoff[i], k1 = a.eoff[i + 1];
-  const int A = a.leaf_of[i], o0 = a.p2p_off[A], o1 = a.p2p_off[A + 1];
-  int m = 0;
-  for (int k = k0; k < k1; ++k) {
-    if (!excl_in_near(a, i, k0, k, o0, o1)) continue;
-    if (off) out[off[i] + m] = a.eidx[k];
-    ++m;
-  }
-  if (!off) out[i] = m;
-}
-
-// Takes the excluded near-field pairs out of a near-field sum that included them: for each site
-// i and each distinct exclusion partner e != i whose leaf is in the near list of i's leaf, out[i]
-// -= pair(i, e), evaluated as the staged kernel does (same record, same arithmetic; FP32: offsets
-// from i's leaf centre). K right-hand sides as in the staged kernel. LISTED: a.eoff / a.eidx hold
-// those partners already (FmmState::xn_off / xn_idx), so no partner is tested here. SYM: the
-// symmetric near field evaluated a pair across leaves once, from the lower leaf (its centre, its site
-// as the target); such a pair is evaluated here the same way, so that it is taken out as it was added.
-template <typename R, bool DAMP, typename MU4, bool B2 = false, int K = 1, bool LISTED = false, bool SYM = false>
-__global__ __launch_bounds__(256) void k_fmm_excl_sub(NearArgs a, const MU4* __restrict__ mu4) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
-  const int k0 = a.eoff[i], k1 = a.eoff[i + 1];
+  const int k0 = sk.off[i], k1 = sk.off[i + 1];
   if (k0 == k1) return;
   const int n      = a.n;
   const int A      = a.leaf_of[i];
-  const int o0 = LISTED ? 0 : a.p2p_off[A], o1 = LISTED ? 0 : a.p2p_off[A + 1];
   const double4 pi = a.pos4[i];
-  const double cax = a.cx[A], cay = a.cy[A], caz = a.cz[A];
-  const R xi = sizeof(R) == 8 ? (R)pi.x : (R)(pi.x - cax);
-  const R yi = sizeof(R) == 8 ? (R)pi.y : (R)(pi.y - cay);
-  const R zi = sizeof(R) == 8 ? (R)pi.z : (R)(pi.z - caz);
+  const double cx = a.cx[A], cy = a.cy[A], cz = a.cz[A];
   const R di = DAMP ? staged_di<R, B2>(a.damping, pi.w) : R(0);
-  R f[3 * K];
-#pragma unroll
-  for (int c = 0; c < 3 * K; ++c) f[c] = R(0);
+  R f[3]     = {R(0), R(0), R(0)};
   for (int k = k0; k < k1; ++k) {
-    if (!LISTED && !excl_in_near(a, i, k0, k, o0, o1)) continue;
-    const int e      = a.eidx[k];
+    const unsigned v = sk.ent[k];
+    const int e      = (int)(v & kSkipSite);
+    if (((v & kSkipKeep) != 0) != KEEP || !leaves_near(a, A, a.leaf_of[e])) continue;
     const double4 pj = a.pos4[e];
-    StagedRec<R, K> r;
-#pragma unroll
-    for (int q = 0; q < K; ++q) {
-      const MU4 mj   = mu4[(size_t)q * n + e];
-      r.m[3 * q]     = (R)mj.x;
-      r.m[3 * q + 1] = (R)mj.y;
-      r.m[3 * q + 2] = (R)mj.z;
+    const MU4 mj     = mu4[e];
+    StagedRec<R, 1> r;
+    r.s    = (R)pj.w;
+    r.m[0] = (R)mj.x;
+    r.m[1] = (R)mj.y;
+    r.m[2] = (R)mj.z;
+    R d[3];
+    if (sizeof(R) == 8 || KEEP) {
+      d[0] = (R)(pi.x - pj.x);
+      d[1] = (R)(pi.y - pj.y);
+      d[2] = (R)(pi.z - pj.z);
+    } else {  // as the staged form: offsets from the leaf's centre
+      d[0] = (R)(pi.x - cx) - (R)(pj.x - cx);
+      d[1] = (R)(pi.y - cy) - (R)(pj.y - cy);
+      d[2] = (R)(pi.z - cz) - (R)(pj.z - cz);
     }
-    if (SYM) {
-      const int Ae = a.leaf_of[e];
-      if (Ae < A) {  // e was the target: positions from its leaf's centre, its damping rate, i's scale
-        const double cx = a.cx[Ae], cy = a.cy[Ae], cz = a.cz[Ae];
-        r.x = sizeof(R) == 8 ? (R)pi.x : (R)(pi.x - cx);
-        r.y = sizeof(R) == 8 ? (R)pi.y : (R)(pi.y - cy);
-        r.z = sizeof(R) == 8 ? (R)pi.z : (R)(pi.z - cz);
-        r.s = (R)pi.w;
-        const R ex = sizeof(R) == 8 ? (R)pj.x : (R)(pj.x - cx);
-        const R ey = sizeof(R) == 8 ? (R)pj.y : (R)(pj.y - cy);
-        const R ez = sizeof(R) == 8 ? (R)pj.z : (R)(pj.z - cz);
-        const R de = DAMP ? staged_di<R, B2>(a.damping, pj.w) : R(0);
-        staged_pair<R, DAMP, (sizeof(R) == 4 && B2), K>(ex, ey, ez, de, r, f);
-        continue;
-      }
-    }
-    r.x = sizeof(R) == 8 ? (R)pj.x : (R)(pj.x - cax);
-    r.y = sizeof(R) == 8 ? (R)pj.y : (R)(pj.y - cay);
-    r.z = sizeof(R) == 8 ? (R)pj.z : (R)(pj.z - caz);
-    r.s = (R)pj.w;
-    staged_pair<R, DAMP, (sizeof(R) == 4 && B2), K>(xi, yi, zi, di, r, f);
+    staged_pair<R, DAMP, B2, 1, false, !KEEP>(d[0], d[1], d[2], di, r, f);
   }
-#pragma unroll
-  for (int q = 0; q < K; ++q) {
-    const size_t o = 3 * (size_t)n * q;
-    a.out[o + i] -= (double)f[3 * q];
-    a.out[o + n + i] -= (double)f[3 * q + 1];
-    a.out[o + 2 * (size_t)n + i] -= (double)f[3 * q + 2];
-  }
+  const double sg = KEEP ? 1.0 : -1.0;
+  a.out[i] += sg * (double)f[0];
+  a.out[n + i] += sg * (double)f[1];
+  a.out[2 * (size_t)n + i] += sg * (double)f[2];
 }
+
+// Skip list entries of a work item's targets i0 .. i0 + T - 1 and, for a stage of 64 sources, one per lane, which
+// targets leave the lane's source out. The first 64 entries stand in wavefront-private LDS, each with the target it
+// belongs to (in registers they would cost the tiled direct form its second block on a CU); any beyond are read
+// from memory, one after another. A kernel keeps what it needs to tell which of them can meet a stage (its lane's).
+struct ItemSkips {
+  const int2* lds;
+  SkipLists sk;
+  int i0, off = 0, n = 0;
+  // this lane's entry goes to ent (lane < n)
+  __device__ __forceinline__ ItemSkips(const SkipLists& s, int i0_, int T, int lane, int2* mem, unsigned& ent)
+      : lds(mem), sk(s), i0(i0_) {
+    ent = 0;
+    if (!sk.off || T <= 0) return;
+    off = __builtin_amdgcn_readfirstlane(sk.off[i0]);
+    n   = __builtin_amdgcn_readfirstlane(sk.off[i0 + T]) - off;
+    if (lane < n) {
+      int t = 0;
+      ent   = sk.ent[off + lane];
+      while (sk.off[i0 + t + 1] - off <= lane) ++t;
+      mem[lane] = make_int2((int)ent, t);
+    }
+    wave_lds_barrier();
+  }
+  // Bit t of the result: target t skips site j, by the entries of lanes m (and all beyond 64). OWN: entries
+  // marked kSkipKeep do not count.
+  template <bool OWN>
+  __device__ __forceinline__ unsigned of(int j, unsigned long long m) const {
+    unsigned skip = 0;
+    auto take     = [&](unsigned v, int t) {
+      if ((int)(v & kSkipSite) == j && !(OWN && (v & kSkipKeep))) skip |= 1u << t;
+    };
+    while (m) {
+      const int2 v = lds[__ffsll(m) - 1];
+      m &= m - 1;
+      take((unsigned)v.x, v.y);
+    }
+    int t = 0;
+    for (int k = 64; k < n; ++k) {
+      while (sk.off[i0 + t + 1] - off <= k) ++t;
+      take(sk.ent[off + k], t);
+    }
+    return skip;
+  }
+};
 
 // out += L2P of each site's leaf expansion (the far-field term when it runs beside the near field)
 // (grid.y = right-hand side: L + y lstride, out + 3 y n)
@@ -1729,48 +1725,19 @@ inline void ensure_posf4(System& S) {
                      T.leaf_of.p, T.cx.p, T.cy.p, T.cz.p, F.posf4.p);
 }
 
-// The exclusion partners whose pairs the near field adds (k_excl_near), per site, once per tree;
-// nothing when the system has no exclusions. Allocates: the CG reserves it before any capture.
-inline void ensure_excl_near(System& S) {
-  FmmState& F = *S.fmm;
-  if (F.xn_built || !S.excl_off.p) return;
-  const Octree& T = S.tree;
-  NearArgs a{};
-  a.leaf_of = T.leaf_of.p;
-  a.p2p_off = T.p2p_off.p;
-  a.p2p_src = T.p2p_src.p;
-  a.eoff    = S.excl_off.p;
-  a.eidx    = S.excl_idx.p;
-  a.n       = S.n;
-  const dim3 g(ceil_div(S.n, 256)), b(256);
-  dbuf<int> cnt;
-  cnt.alloc((size_t)S.n + 1);
-  F.xn_off.alloc((size_t)S.n + 1);
-  CPPE_HIP_CHECK(hipMemsetAsync(cnt.p + S.n, 0, sizeof(int), S.stream));
-  hipLaunchKernelGGL(k_excl_near, g, b, 0, S.stream, a, nullptr, cnt.p);
-  device_scan(S, cnt.p, F.xn_off.p, S.n + 1);
-  int tot = 0;
-  CPPE_HIP_CHECK(hipMemcpy(&tot, F.xn_off.p + S.n, sizeof(int), hipMemcpyDeviceToHost));
-  F.xn_idx.alloc((size_t)std::max(tot, 1));
-  hipLaunchKernelGGL(k_excl_near, g, b, 0, S.stream, a, F.xn_off.p, F.xn_idx.p);
-  CPPE_HIP_CHECK(hipStreamSynchronize(S.stream));
-  F.xn_built = true;
-}
-
-// k_fmm_excl_sub over the listed partners (ensure_excl_near)
-template <typename R, bool DAMP, typename MU4, int K, bool SYM = false>
-void launch_excl_sub(System& S, const NearArgs& a, const MU4* mu4, bool b2, hipStream_t st) {
+// k_fmm_skip_fix after a pass that KEEP describes there (nothing without exclusions).
+template <typename R, bool DAMP, bool KEEP, typename MU4>
+void launch_skip_fix(System& S, const NearArgs& a, const MU4* mu4, bool b2, hipStream_t st) {
   if (!a.eoff) return;
-  ensure_excl_near(S);
-  NearArgs ax             = a;
-  ax.eoff                 = S.fmm->xn_off.p;
-  ax.eidx                 = S.fmm->xn_idx.p;
-  constexpr bool kB2      = sizeof(R) == 4 && DAMP;
+  build_pair_skips(S);
+  if (KEEP && !S.skips.one_way) return;
+  constexpr bool kB2 = sizeof(R) == 4 && DAMP;
+  const SkipLists sk = S.skips.lists();
   const dim3 g(ceil_div(S.n, 256)), b(256);
   if (b2)
-    hipLaunchKernelGGL((k_fmm_excl_sub<R, DAMP, MU4, kB2, K, true, SYM>), g, b, 0, st, ax, mu4);
+    hipLaunchKernelGGL((k_fmm_skip_fix<R, DAMP, kB2, KEEP, MU4>), g, b, 0, st, a, sk, mu4);
   else
-    hipLaunchKernelGGL((k_fmm_excl_sub<R, DAMP, MU4, false, K, true, SYM>), g, b, 0, st, ax, mu4);
+    hipLaunchKernelGGL((k_fmm_skip_fix<R, DAMP, false, KEEP, MU4>), g, b, 0, st, a, sk, mu4);
 }
 
 void ensure_clusters(System& S);  // fmm.hip
@@ -1808,6 +1775,7 @@ inline void ensure_sym_trec(System& S, int prec, double damping) {
 inline SymLists& ensure_sym(System& S, int prec, int ts, double damping) {
   FmmState& F = *S.fmm;
   SymLists& Y = build_sym_lists(S, prec, ts);
+  build_pair_skips(S);
   ensure_sym_trec(S, prec, damping);
   if (prec)
     ensure_buf(F.rev32, (size_t)std::max<long long>(Y.nrev, 1));
@@ -1849,6 +1817,7 @@ inline FmmState::DSym& ensure_dsym(System& S, int prec, int ts, double damping) 
   FmmState& F       = *S.fmm;
   FmmState::DSym& D = F.dsym[prec];
   ensure_sym_trec(S, prec, damping);
+  build_pair_skips(S);
   if (D.ts != ts) {
     const int n = S.n, TB = kDSymW * ts;
     const int ntile  = (n + TB - 1) / TB;
@@ -1930,7 +1899,7 @@ void launch_direct_sym(System& S, const NearArgs& a, const MU4* mu4, const R* L,
   constexpr bool kB2 = prec && DAMP;
   const bool b2      = kB2 && S.all_damped;
   hipStream_t st     = S.stream;
-  const DSymArgs da{D.items.p, D.nitems, S.n, D.fwd_off.p, D.c[0], D.c[1], D.c[2]};
+  const DSymArgs da{D.items.p, D.nitems, S.n, D.fwd_off.p, D.c[0], D.c[1], D.c[2], S.skips.lists()};
   R *fwd, *rev;
   if constexpr (prec) {
     fwd = F.dfwd32.p;
@@ -1953,30 +1922,19 @@ void launch_direct_sym(System& S, const NearArgs& a, const MU4* mu4, const R* L,
                        mu4, fwd, rev);
   }
   if (S.prof) CPPE_HIP_CHECK(hipEventRecord(S.prof[7], st));
-  // the gather ends the apply: exclusions, alpha^-1 mu and, when the CG step asked, its partials
-  NearArgs ax = a;
-  if (a.eoff) {
-    ensure_excl_near(S);
-    ax.eoff = F.xn_off.p;
-    ax.eidx = F.xn_idx.p;
-  }
-  auto gather = [&](auto lanes, auto sites, auto bb) {
+  // the gather ends the apply: alpha^-1 mu and, when the CG step asked, its partials
+  const bool more = with_l2p || S.skips.one_way;
+  auto gather     = [&](auto lanes, auto sites) {
     constexpr int G = decltype(lanes)::value, SB = decltype(sites)::value;
     const int nb       = ceil_div(S.n, SB);
-    const L2pDots dots = with_l2p ? L2pDots{} : step_dots(S, a.out, nb);
-    hipLaunchKernelGGL((k_direct_sym_gather<R, DAMP, decltype(bb)::value, G, SB, MU4>), dim3(nb), dim3(SB * G), 0, st,
-                       ax, mu4, da, D.tb, fwd, rev, dots);
+    const L2pDots dots = more ? L2pDots{} : step_dots(S, a.out, nb);
+    hipLaunchKernelGGL((k_direct_sym_gather<R, G, SB>), dim3(nb), dim3(SB * G), 0, st, a, da, D.tb, fwd, rev, dots);
   };
-  auto gather_b = [&](auto bb) {
-    if (S.n < kDSymGatherOne)
-      gather(std::integral_constant<int, 16>{}, std::integral_constant<int, kDotSites>{}, bb);
-    else
-      gather(std::integral_constant<int, 1>{}, std::integral_constant<int, 256>{}, bb);
-  };
-  if (b2)
-    gather_b(std::integral_constant<bool, kB2>{});
+  if (S.n < kDSymGatherOne)
+    gather(std::integral_constant<int, 16>{}, std::integral_constant<int, kDotSites>{});
   else
-    gather_b(std::false_type{});
+    gather(std::integral_constant<int, 1>{}, std::integral_constant<int, 256>{});
+  launch_skip_fix<R, DAMP, true>(S, a, mu4, b2, st);
   if (with_l2p) launch_l2p_add<P, R>(S, L, a.out, st);
 }
 
@@ -2000,7 +1958,7 @@ void launch_near_sym(System& S, const NearArgs& a, const MU4* mu4, const R* L, b
   for (int k = 0; k < splits; ++k) {
     const int i0 = (int)((long long)Y.nitems * k / splits), i1 = (int)((long long)Y.nitems * (k + 1) / splits);
     if (i1 <= i0) continue;
-    const SymArgs sa{Y.items.p + i0, i1 - i0, Y.uoff.p, usp, Y.usrc.p, Y.udst.p};
+    const SymArgs sa{Y.items.p + i0, i1 - i0, Y.uoff.p, usp, Y.usrc.p, Y.udst.p, S.skips.lists()};
     const dim3 g(ceil_div(i1 - i0, block / 64)), b(block);
     if constexpr (prec) {
       if (b2)
@@ -2015,7 +1973,7 @@ void launch_near_sym(System& S, const NearArgs& a, const MU4* mu4, const R* L, b
     }
   }
   if (S.prof) CPPE_HIP_CHECK(hipEventRecord(S.prof[7], st));
-  launch_excl_sub<R, DAMP, MU4, 1, true>(S, a, mu4, b2, st);
+  launch_skip_fix<R, DAMP, true>(S, a, mu4, b2, st);
   launch_sym_gather<P, R>(S, Y, nullptr, a.out);
   if (with_l2p) launch_l2p_add<P, R>(S, L, a.out, st);
 }
@@ -2073,8 +2031,8 @@ void launch_near(System& S, const NearArgs& a, const MU4* mu4, const R* L, bool 
         const int c0 = (int)((long long)ni * k / splits), c1 = (int)((long long)ni * (k + 1) / splits);
         if (c1 <= c0) continue;
         hipLaunchKernelGGL((k_fmm_near_ls<P, R, DAMP, MODE, MU4, decltype(l2p)::value, TS, decltype(bb)::value, K>),
-                           dim3(ceil_div(c1 - c0, block / 64)), dim3(block), 0, st, a, items + c0, c1 - c0, T.xoff.p,
-                           T.xsrc.p, xs, mu4, L, lstride);
+                           dim3(ceil_div(c1 - c0, block / 64)), dim3(block), 0, st, a, S.skips.lists(), items + c0, c1 - c0,
+                           T.xoff.p, T.xsrc.p, T.xspec.p, xs, mu4, L, lstride);
       }
       if (S.prof) CPPE_HIP_CHECK(hipEventRecord(S.prof[7], st));
     };
@@ -2094,7 +2052,6 @@ void launch_near(System& S, const NearArgs& a, const MU4* mu4, const R* L, bool 
       go_ts(std::true_type{});
     else
       go_ts(std::false_type{});
-    launch_excl_sub<R, DAMP, MU4, K>(S, a, mu4, b2, st);
   } else if constexpr (K > 1) {
     throw hip_error("several right-hand sides per launch need a staged near-field variant");
   } else if (var >= 5) {  // 5, 6: staged, chunks of 64, 32 targets
@@ -2134,7 +2091,7 @@ void launch_near(System& S, const NearArgs& a, const MU4* mu4, const R* L, bool 
     else
       go1(std::false_type{});
     if (S.prof) CPPE_HIP_CHECK(hipEventRecord(S.prof[7], st));
-    launch_excl_sub<R, DAMP, MU4, 1>(S, a, mu4, b2, st);
+    launch_skip_fix<R, DAMP, false>(S, a, mu4, b2, st);
   } else if (var == 4) {
     ensure_clusters(S);
     const dim3 g(ceil_div(F.n_clusters, block / 64)), b(block);

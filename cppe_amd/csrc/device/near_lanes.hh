@@ -10,17 +10,19 @@
 // undamped pair. The lanes' fields are summed over the wavefront once per chunk.
 // The records of the next stage and the source index of the one after are loaded while a stage is
 // evaluated. Stages of the list's far class take the undamped pair (xsplit of the precision); excluded
-// pairs are evaluated like all others and taken out afterwards with the same arithmetic
-// (k_fmm_excl_sub), the self pair gives zero. Chunks of a leaf have equal sizes up to one, so that no
+// pairs and the targets themselves are skipped: both stand only in the head of the list (to xspec, the leaf's own sites
+// first), whose stages look for them and have a loop of their own. Chunks of a leaf have equal sizes up to one, so that no
 // short chunk walks the whole list for a few targets.
 // Near field of one apply against the staged form with chunks of 8 (same systems; plus exclusions): FP32
 // 0.156 -> 0.121 ms at 24,000 sites, 0.146 -> 0.123 at 60,000, 0.468 -> 0.388 at 300,000 (chunks of 16);
 // FP64 0.397 -> 0.259, 0.56 -> 0.358, 1.45 -> 1.31 ms (chunks of 4: FP64 accumulators and the prefetched
 // record leave room for more wavefronts then, and the undamped stages drop the exponential).
 template <int P, typename R, bool DAMP, int MODE, typename MU4, bool WITH_L2P, int TS, bool B2, int K>
-__global__ __launch_bounds__(256) void k_fmm_near_ls(NearArgs a, const int4* __restrict__ items, int nitems,
+__global__ __launch_bounds__(256) void k_fmm_near_ls(NearArgs a, SkipLists sk, const int4* __restrict__ items,
+                                                     int nitems,
                                                      const long long* __restrict__ xoff,
                                                      const int* __restrict__ xsrc,
+                                                     const long long* __restrict__ xspec,
                                                      const long long* __restrict__ xsplit,
                                                      const MU4* __restrict__ mu4, const R* __restrict__ L,
                                                      size_t lstride) {
@@ -52,22 +54,24 @@ __global__ __launch_bounds__(256) void k_fmm_near_ls(NearArgs a, const int4* __r
     }
   }
   const long long q0 = xoff[A], q1 = xoff[A + 1];
+  const long long qs = min(q1, q0 + (xspec[A] - q0 + 63) / 64 * 64);  // stages of the head
   const long long qf = DAMP && xsplit ? xsplit[A] : q1;
   constexpr R kFar   = sizeof(R) == 4 ? R(1.0e4) : R(1.0e8);  // lanes past the list: a source far away, no dipole
   double4 pn = make_double4(0.0, 0.0, 0.0, 0.0);
   MU4 mn[K];
-  int jnn     = 0;
+  int jn = -1, jnn = 0;  // source of the record in pn, and of the stage after it
   auto gather = [&](int j) {
+    jn = j;
     pn = a.pos4[j];
 #pragma unroll
     for (int k = 0; k < K; ++k) mn[k] = mu4[(size_t)k * n + j];
   };
   if (lane < q1 - q0) gather(xsrc[q0 + lane]);
   if (lane < q1 - q0 - 64) jnn = xsrc[q0 + 64 + lane];
-  // two loops, not a branch per stage: with both forms of the pair in one loop the compiler keeps the
+  // a loop for each form, not a branch per stage: with two forms of the pair in one loop the compiler keeps the
   // accumulators twice
   long long q = q0;
-  auto walk   = [&](auto far, long long end) {
+  auto walk   = [&](auto far, long long end, auto&& skips) {
     for (; q < end; q += 64) {
       StagedRec<R, K> r;
       r.x = sizeof(R) == 8 ? (R)pn.x : (R)(pn.x - cax);
@@ -80,6 +84,7 @@ __global__ __launch_bounds__(256) void k_fmm_near_ls(NearArgs a, const int4* __r
         r.m[3 * k + 1] = (R)mn[k].y;
         r.m[3 * k + 2] = (R)mn[k].z;
       }
+      const unsigned skip = skips(jn);
       if (q1 - q < 64 && lane >= q1 - q) {
         r.x = r.y = r.z = kFar;
         r.s = R(0);
@@ -90,11 +95,30 @@ __global__ __launch_bounds__(256) void k_fmm_near_ls(NearArgs a, const int4* __r
       if (lane < q1 - q - 128) jnn = xsrc[q + 128 + lane];  // stage s + 2: its source index
 #pragma unroll
       for (int t = 0; t < TS; ++t)
-        if (t < T) staged_pair<R, DAMP, B2, K, decltype(far)::value>(tx[t], ty[t], tz[t], td[t], r, f[t]);
+        if (t < T)
+          staged_pair<R, DAMP, B2, K, decltype(far)::value, false>(tx[t] - r.x, ty[t] - r.y, tz[t] - r.z, td[t], r, f[t],
+                                                                   skip >> t & 1u);
     }
   };
-  walk(std::false_type{}, min(q1, qf));
-  if (DAMP) walk(std::true_type{}, q1);
+  {  // the head: own sites stand at q0 + (site - start), partners in other leaves behind them
+    const int ia = __builtin_amdgcn_readfirstlane(a.start[A]), na = __builtin_amdgcn_readfirstlane(a.count[A]);
+    __shared__ int2 mem[4][64];
+    unsigned ent;
+    const ItemSkips its(sk, i0, T, lane, mem[threadIdx.x >> 6], ent);
+    const int at                   = (int)(ent & kSkipSite) - ia;
+    const bool inside              = lane < its.n && (unsigned)at < (unsigned)na;
+    const unsigned long long other = __ballot(lane < its.n && !inside);
+    walk(std::false_type{}, qs, [&](int j) {
+      const int qr               = (int)(q - q0);
+      const unsigned long long m = other | __ballot(inside && (unsigned)(at - qr) < 64u);
+      unsigned s                 = (unsigned)(j - i0) < (unsigned)T ? 1u << (j - i0) : 0u;
+      if (m != 0 || its.n > 64) s |= its.template of<true>(j, m);
+      return s;
+    });
+  }
+  const auto none = [](int) { return 0u; };
+  walk(std::false_type{}, min(q1, qf), none);
+  if (DAMP) walk(std::true_type{}, q1, none);
   double F[3 * K];
 #pragma unroll
   for (int c = 0; c < 3 * K; ++c) F[c] = 0.0;

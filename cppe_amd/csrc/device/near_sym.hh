@@ -20,9 +20,8 @@
 // gather kernel adds, per site of B, its blocks in that order, then the L2P term: every sum has a
 // fixed order, and no atomics are used, so applies are bit-reproducible.
 //
-// Exclusions: excluded pairs are evaluated like every other pair and taken out afterwards per
-// site by k_fmm_excl_sub (the field at the lower leaf's site with the same arithmetic; at the other
-// site to the rounding of the precision).
+// Exclusions: a pair that either side excludes is skipped in both directions (and so is a target with itself); where
+// only one side excludes it, k_fmm_skip_fix adds the other side's field afterwards.
 //
 // Included by fmm_impl.hh inside namespace cppe_dev (uses NearArgs, the staged pair arithmetic
 // and the FMM operators).
@@ -35,6 +34,7 @@ struct SymArgs {
   const long long* usplit;    // per cell (FP32): first entry whose stages may use the undamped pair
   const int* usrc;            // upper list: source site
   const int2* udst;           // upper list: (reverse slot of chunk 0 / component x, |B|)
+  SkipLists sk;
 };
 
 template <typename R>
@@ -47,10 +47,10 @@ struct SymTarget {
   SymVec4<R> p, m;
 };
 
-// Geometry once, field at both ends: f += T(d) mu_s, r += T(d) mu_t.
+// Geometry once, field at both ends: f += T(d) mu_s, r += T(d) mu_t (skip: neither).
 template <typename R, bool DAMP, bool B2, bool FAR>
 __device__ __forceinline__ void sym_pair(const SymTarget<R>& t, R xs, R ys, R zs, R ss, R mxs, R mys, R mzs, R& fx,
-                                         R& fy, R& fz, R& rx, R& ry, R& rz) {
+                                         R& fy, R& fz, R& rx, R& ry, R& rz, bool skip) {
   const SymVec4<R> tp = t.p, tm = t.m;
   const R dx = tp.x - xs, dy = tp.y - ys, dz = tp.z - zs;
   if constexpr (FAR && sizeof(R) == 4) {
@@ -60,7 +60,7 @@ __device__ __forceinline__ void sym_pair(const SymTarget<R>& t, R xs, R ys, R zs
     acc_far_f32(ri3, m3, dx, dy, dz, tm.x, tm.y, tm.z, rx, ry, rz);
   } else {
     R c3, cf;
-    staged_geo<R, DAMP, B2, FAR>(dx, dy, dz, tp.w * ss, c3, cf);
+    staged_geo<R, DAMP, B2, FAR, false>(dx, dy, dz, tp.w * ss, c3, cf, skip);
     acc_m1(c3, cf, dx, dy, dz, mxs, mys, mzs, fx, fy, fz);
     acc_m1(c3, cf, dx, dy, dz, tm.x, tm.y, tm.z, rx, ry, rz);
   }
@@ -136,20 +136,30 @@ __global__ __launch_bounds__(256) void k_fmm_near_sym(NearArgs a, SymArgs b, con
     tg[lane].m    = SymVec4<R>{(R)mt.x, (R)mt.y, (R)mt.z, R(0)};
   }
   wave_lds_barrier();
-  // A's own sites: ordered pairs, field at the item's targets only (the self pair gives zero)
+  // skip list entries of the item's targets: partners in the leaf stand at e0 + (site - start); of the others only
+  // those in leaves above A are sources here
+  __shared__ int2 mem[4][64];
+  unsigned ent;
+  const ItemSkips its(b.sk, i0, T, lane, mem[threadIdx.x >> 6], ent);
+  const int partner              = (int)(ent & kSkipSite), at = partner - a.start[A];
+  const bool inside              = lane < its.n && (unsigned)at < (unsigned)a.count[A];
+  const unsigned long long above = __ballot(lane < its.n && !inside && a.leaf_of[partner] > A);
+  // A's own sites: ordered pairs, field at the item's targets only
   for (long long q0 = e0; q0 < es; q0 += 64) {
     const bool act = q0 + lane < es;
     R xs, ys, zs, ss, mx, my, mz;
     const int j = a.start[A] + (int)(q0 - e0) + lane;
     convert(act ? a.pos4[j] : make_double4(0.0, 0.0, 0.0, 0.0), act ? mu4[j] : MU4{}, act, xs, ys, zs, ss, mx, my,
             mz);
+    unsigned skip = (unsigned)(j - i0) < (unsigned)T ? 1u << (j - i0) : 0u;
+    skip |= its.template of<false>(j, __ballot(inside && (unsigned)(at - (int)(q0 - e0)) < 64u));
 #pragma unroll
     for (int t = 0; t < TS; ++t) {
       if (t < T) {
         const SymVec4<R> tp = tg[t].p;
         const R dx = tp.x - xs, dy = tp.y - ys, dz = tp.z - zs;
         R c3, cf;
-        staged_geo<R, DAMP, B2, false>(dx, dy, dz, tp.w * ss, c3, cf);
+        staged_geo<R, DAMP, B2, false, false>(dx, dy, dz, tp.w * ss, c3, cf, skip >> t & 1u);
         acc_m1(c3, cf, dx, dy, dz, mx, my, mz, f[t][0], f[t][1], f[t][2]);
       }
     }
@@ -159,12 +169,12 @@ __global__ __launch_bounds__(256) void k_fmm_near_sym(NearArgs a, SymArgs b, con
   double4 pn = make_double4(0.0, 0.0, 0.0, 0.0);
   MU4 mn{};
   int2 dn = make_int2(0, 0), dnn = make_int2(0, 0);
-  int jnn = 0;
+  int jn = -1, jnn = 0;
   if (es + lane < e1) {
-    const int j0 = b.usrc[es + lane];
+    jn = b.usrc[es + lane];
     dn = b.udst[es + lane];
-    pn = a.pos4[j0];
-    mn = mu4[j0];
+    pn = a.pos4[jn];
+    mn = mu4[jn];
   }
   if (es + 64 + lane < e1) {
     jnn = b.usrc[es + 64 + lane];
@@ -175,7 +185,10 @@ __global__ __launch_bounds__(256) void k_fmm_near_sym(NearArgs a, SymArgs b, con
     R xs, ys, zs, ss, mx, my, mz;
     convert(pn, mn, act, xs, ys, zs, ss, mx, my, mz);
     const int2 dd = dn;
+    unsigned skip = 0;
+    if (above != 0 || its.n > 64) skip = its.template of<false>(jn, above);
     if (q0 + 64 + lane < e1) {  // stage s + 1
+      jn = jnn;
       pn = a.pos4[jnn];
       mn = mu4[jnn];
       dn = dnn;
@@ -188,11 +201,13 @@ __global__ __launch_bounds__(256) void k_fmm_near_sym(NearArgs a, SymArgs b, con
     if (q0 >= ef) {  // every pair of the stage beyond the precision's damping cutoff (uniform)
 #pragma unroll
       for (int t = 0; t < TS; ++t)
-        if (t < T) sym_pair<R, DAMP, B2, true>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz);
+        if (t < T) sym_pair<R, DAMP, B2, true>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz, false);
     } else {
 #pragma unroll
       for (int t = 0; t < TS; ++t)
-        if (t < T) sym_pair<R, DAMP, B2, false>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz);
+        if (t < T)
+          sym_pair<R, DAMP, B2, false>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz,
+                                       skip >> t & 1u);
     }
     if (act) {
       const int o = dd.x + q * 3 * dd.y;
@@ -277,6 +292,7 @@ struct DSymArgs {
   int nitems, n;
   const long long* fwd_off;  // per tile: first forward slot
   double cx, cy, cz;         // the leaf's centre (FP32 offsets)
+  SkipLists sk;
 };
 
 __device__ __forceinline__ long long dsym_rev_block(int J, int I, int TB) {
@@ -309,6 +325,10 @@ __global__ __launch_bounds__(64 * W) void k_direct_sym(NearArgs a, DSymArgs b, c
   R f[TS][3];
 #pragma unroll
   for (int t = 0; t < TS; ++t) f[t][0] = f[t][1] = f[t][2] = R(0);
+  __shared__ int2 mem[W][64];
+  unsigned ent;
+  const ItemSkips its(b.sk, t0, T, lane, mem[wv], ent);
+  const int partner = lane < its.n ? (int)(ent & kSkipSite) : -1;
   int buf = 0;
   for (long long q0 = s0; q0 < s1; q0 += 64) {
     const long long j = q0 + lane;
@@ -325,14 +345,18 @@ __global__ __launch_bounds__(64 * W) void k_direct_sym(NearArgs a, DSymArgs b, c
       my = (R)mj.y;
       mz = (R)mj.z;
     }
-    if (diag) {  // ordered pairs inside the tile (the self pair gives zero)
+    unsigned skip = 0;  // targets that leave this source out
+    const unsigned long long in = __ballot(partner >= q0 && partner < q0 + 64);
+    if (in != 0 || its.n > 64) skip = its.template of<false>((int)j, in);
+    if (diag) {  // ordered pairs inside the tile
+      if (j >= t0 && j < t0 + T) skip |= 1u << (int)(j - t0);
 #pragma unroll
       for (int t = 0; t < TS; ++t) {
         if (t < T) {
           const SymVec4<R> tp = tg[t].p;
           const R dx = tp.x - xs, dy = tp.y - ys, dz = tp.z - zs;
           R c3, cf;
-          staged_geo<R, DAMP, B2, false>(dx, dy, dz, tp.w * ss, c3, cf);
+          staged_geo<R, DAMP, B2, false, false>(dx, dy, dz, tp.w * ss, c3, cf, skip >> t & 1u);
           acc_m1(c3, cf, dx, dy, dz, mx, my, mz, f[t][0], f[t][1], f[t][2]);
         }
       }
@@ -341,7 +365,9 @@ __global__ __launch_bounds__(64 * W) void k_direct_sym(NearArgs a, DSymArgs b, c
     R rx = R(0), ry = R(0), rz = R(0);
 #pragma unroll
     for (int t = 0; t < TS; ++t)
-      if (t < T) sym_pair<R, DAMP, B2, false>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz);
+      if (t < T)
+        sym_pair<R, DAMP, B2, false>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz,
+                                     skip >> t & 1u);
     red[buf][wv][0][lane] = rx;
     red[buf][wv][1][lane] = ry;
     red[buf][wv][2][lane] = rz;
@@ -373,42 +399,17 @@ __global__ __launch_bounds__(64 * W) void k_direct_sym(NearArgs a, DSymArgs b, c
   }
 }
 
-// The exclusion partners of a site taken out of a near-field sum that included them: partners
-// eidx[eoff[i] ..] (FmmState::xn_idx), every pair with the arithmetic of the staged kernel.
-template <typename R, bool DAMP, bool B2, typename MU4>
-__device__ __forceinline__ void excl_pairs(const NearArgs& a, const MU4* __restrict__ mu4, int i, int k, double cax,
-                                           double cay, double caz, R* f) {
-  const double4 pi = a.pos4[i];
-  const int e      = a.eidx[k];
-  const double4 pj = a.pos4[e];
-  const MU4 mj     = mu4[e];
-  StagedRec<R, 1> r;
-  r.x = sizeof(R) == 8 ? (R)pj.x : (R)(pj.x - cax);
-  r.y = sizeof(R) == 8 ? (R)pj.y : (R)(pj.y - cay);
-  r.z = sizeof(R) == 8 ? (R)pj.z : (R)(pj.z - caz);
-  r.s = (R)pj.w;
-  r.m[0] = (R)mj.x;
-  r.m[1] = (R)mj.y;
-  r.m[2] = (R)mj.z;
-  const R xi = sizeof(R) == 8 ? (R)pi.x : (R)(pi.x - cax);
-  const R yi = sizeof(R) == 8 ? (R)pi.y : (R)(pi.y - cay);
-  const R zi = sizeof(R) == 8 ? (R)pi.z : (R)(pi.z - caz);
-  const R di = DAMP ? staged_di<R, B2>(a.damping, pi.w) : R(0);
-  staged_pair<R, DAMP, (sizeof(R) == 4 && B2), 1>(xi, yi, zi, di, r, f);
-}
-
-// out = (the tile's forward blocks) + (reverse blocks from the tiles below) + alpha^-1 mu - excluded
-// pairs. G lanes per site: lane g adds the blocks g, g + G, ... of each kind and takes the exclusion
-// partners g, g + G, ...; the lanes' sums are combined by an xor-shuffle tree, so every sum has a
-// fixed order. A block owns SB consecutive sites (G x SB threads), and with d.p set it also writes
+// out = (the tile's forward blocks) + (reverse blocks from the tiles below) + alpha^-1 mu.
+// G lanes per site: lane g adds the blocks g, g + G, ... of each kind; the lanes' sums are combined by an
+// xor-shuffle tree, so every sum has a fixed order. A block owns SB consecutive sites (G x SB threads), and with d.p set it also writes
 // their partials p.out and out.out (one kernel then ends the apply and starts the step: on small
 // systems each launch costs as much as the sums).
 // G = 16, SB = 64 where one thread per site would leave the device idle and run a chain of n / TB
 // dependent adds (3,000 sites: 12 blocks, 94 reverse blocks a site); G = 1 once the sites alone fill it.
-template <typename R, bool DAMP, bool B2, int G, int SB, typename MU4>
-__global__ __launch_bounds__(SB * G) void k_direct_sym_gather(NearArgs a, const MU4* __restrict__ mu4, DSymArgs b,
-                                                               int TB, const R* __restrict__ fwd,
-                                                               const R* __restrict__ rev, L2pDots d) {
+template <typename R, int G, int SB>
+__global__ __launch_bounds__(SB * G) void k_direct_sym_gather(NearArgs a, DSymArgs b, int TB,
+                                                               const R* __restrict__ fwd, const R* __restrict__ rev,
+                                                               L2pDots d) {
   const int n  = a.n;
   const int i  = blockIdx.x * SB + threadIdx.x / G;
   const int gl = threadIdx.x % G;
@@ -429,13 +430,6 @@ __global__ __launch_bounds__(SB * G) void k_direct_sym_gather(NearArgs a, const 
       g[0] += (double)q[0];
       g[1] += (double)q[TB];
       g[2] += (double)q[2 * TB];
-    }
-    if (a.eoff) {
-      R f[3] = {R(0), R(0), R(0)};
-      for (int k = a.eoff[i] + gl; k < a.eoff[i + 1]; k += G)
-        excl_pairs<R, DAMP, B2>(a, mu4, i, k, b.cx, b.cy, b.cz, f);
-#pragma unroll
-      for (int c = 0; c < 3; ++c) g[c] -= (double)f[c];
     }
   }
 #pragma unroll

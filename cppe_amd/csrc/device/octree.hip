@@ -599,36 +599,113 @@ __global__ void k_xcount(int ncells, const int* __restrict__ off, const int* __r
   xcnt[c] = t;
 }
 
+// Entry of leaf A in the near list of leaf B (sorted by source leaf); without one, where it would stand.
+__device__ __forceinline__ int near_entry(const int* __restrict__ off, const int* __restrict__ src, int B, int A) {
+  int lo = off[B], hi = off[B + 1];
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (src[mid] < A)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  return lo;
+}
+
+// Whether site e is among the exclusion partners eidx[eoff[i] ..] of site i.
+__device__ __forceinline__ bool lists_partner(const int* __restrict__ eoff, const int* __restrict__ eidx, int i, int e) {
+  for (int k = eoff[i]; k < eoff[i + 1]; ++k)
+    if (eidx[k] == e) return true;
+  return false;
+}
+
+// Skip lists: per site the partners a near field leaves out, from either side's exclusions. A site's exclusions
+// count for the field at that site alone (fmm/calculate.cc:205-225); a partner that only lists the site from its
+// own side is marked kSkipKeep: the field at the site keeps that pair. Thread per site, cur[e] the entries
+// of site e so far: with ent null they are counted. one_way is set when a partner is marked.
+__global__ __launch_bounds__(256) void k_pair_skips(int n, const int* __restrict__ eoff, const int* __restrict__ eidx,
+                                                    int* __restrict__ cur, unsigned* __restrict__ ent,
+                                                    int* __restrict__ one_way) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  for (int k = eoff[i]; k < eoff[i + 1]; ++k) {
+    const int e = eidx[k];
+    if (e < 0 || e == i) continue;
+    bool again = false;
+    for (int q = eoff[i]; q < k; ++q) again = again || eidx[q] == e;
+    if (again) continue;
+    const int at = atomicAdd(&cur[i], 1);
+    if (ent) ent[at] = (unsigned)e;
+    if (lists_partner(eoff, eidx, e, i)) continue;
+    *one_way     = 1;
+    const int to = atomicAdd(&cur[e], 1);
+    if (ent) ent[to] = (unsigned)i | kSkipKeep;
+  }
+}
+
+void build_pair_skips(System& S) {
+  PairSkips& K = S.skips;
+  if (K.built || !S.excl_off.p) return;
+  hipStream_t st = S.stream;
+  const dim3 g(ceil_div(S.n, 256)), b(256);
+  dbuf<int> cur, flag;
+  cur.alloc((size_t)S.n + 1);
+  flag.alloc(1);
+  CPPE_HIP_CHECK(hipMemsetAsync(cur.p, 0, sizeof(int) * ((size_t)S.n + 1), st));
+  CPPE_HIP_CHECK(hipMemsetAsync(flag.p, 0, sizeof(int), st));
+  K.off.alloc((size_t)S.n + 1);
+  hipLaunchKernelGGL(k_pair_skips, g, b, 0, st, S.n, S.excl_off.p, S.excl_idx.p, cur.p, nullptr, flag.p);
+  int one_way = 0, total = 0;
+  CPPE_HIP_CHECK(hipMemcpyAsync(&one_way, flag.p, sizeof(int), hipMemcpyDeviceToHost, st));
+  device_scan(S, cur.p, K.off.p, S.n + 1);
+  CPPE_HIP_CHECK(hipMemcpyAsync(&total, K.off.p + S.n, sizeof(int), hipMemcpyDeviceToHost, st));
+  CPPE_HIP_CHECK(hipMemcpyAsync(cur.p, K.off.p, sizeof(int) * (size_t)S.n, hipMemcpyDeviceToDevice, st));
+  CPPE_HIP_CHECK(hipStreamSynchronize(st));
+  K.ent.alloc((size_t)std::max(total, 1));
+  hipLaunchKernelGGL(k_pair_skips, g, b, 0, st, S.n, S.excl_off.p, S.excl_idx.p, cur.p, K.ent.p, flag.p);
+  CPPE_HIP_CHECK(hipStreamSynchronize(st));  // before the scratch is released
+  K.one_way = one_way != 0;
+  K.built   = true;
+}
+
 // Every entry of a cell's expanded near list in near-list order, one block per cell: the source site with
-// its class in the two top bits. The class is that of the smallest Thole argument v = damping s_i s_j R_ij
-// over the leaf's own sites i (exact, FP64): 0: v < 18, 1: 18 <= v < 40, 2: v >= 40 (a small margin above
-// each bound). Undamped sites (s = 0) and the leaf's own sites (the site itself is among the targets, R
-// = 0) give class 0 without the search, so one-leaf (direct-summation) systems cost O(n) here. The near
+// its class in the top bits. XC_OWN: the leaf's own sites. XC_PARTNER: sites of other leaves that the skip list of an
+// own site names. The others by the smallest Thole argument v = damping s_i s_j R_ij
+// over the leaf's own sites i (exact, FP64): XC_NEAR: v < 18, XC_MID: 18 <= v < 40, XC_FAR: v >= 40 (a small
+// margin above each bound). Undamped sites (s = 0) are XC_NEAR without the search, so are one-leaf
+// (direct-summation) systems, all of whose sites are own, and cost O(n) here. The near
 // leaves are taken 256 at a time (prefix sums of their sizes in LDS), the entries 64 at a time by the
 // block's wavefronts, with the leaf's sites in LDS; a wavefront leaves the search once all its entries
-// are of class 0. Per class 0 and 1 the cell's totals go to the splits.
-constexpr int kXclsShift = 30;
+// are of class XC_NEAR. The ends of the classes (totals over the cell) go to ends.
+enum XClass : unsigned { XC_OWN = 0, XC_PARTNER, XC_NEAR, XC_MID, XC_FAR, XC_COUNT };
+constexpr int kXclsShift = 29;
+constexpr unsigned kXclsSite = (1u << kXclsShift) - 1u;
+// ends of the classes XC_OWN, XC_PARTNER, XC_NEAR and XC_MID in the ordered list
+struct XEnds {
+  long long *own, *spec, *s32, *s64;
+};
 __global__ __launch_bounds__(256) void k_xclass(const int* __restrict__ off, const int* __restrict__ src,
                                                 const int* __restrict__ start, const int* __restrict__ count,
-                                                const double* __restrict__ x, const double* __restrict__ y,
-                                                const double* __restrict__ z, const double* __restrict__ s,
-                                                double damping, const long long* __restrict__ xoff,
-                                                unsigned* __restrict__ ent, long long* __restrict__ xs64,
-                                                long long* __restrict__ xs32) {
+                                                const int* __restrict__ leaf_of, const double* __restrict__ x,
+                                                const double* __restrict__ y, const double* __restrict__ z,
+                                                const double* __restrict__ s, double damping, SkipLists sk,
+                                                const long long* __restrict__ xoff, unsigned* __restrict__ ent,
+                                                XEnds ends) {
   __shared__ double4 own[256];
-  __shared__ int pre[256], st[256], part[4], n01[2];
+  __shared__ int pre[256], st[256], part[4], num[XC_COUNT];
   const int c = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int o0 = off[c], o1 = off[c + 1];
   if (o0 == o1) {
-    if (tid == 0) xs32[c] = xs64[c] = xoff[c];
+    if (tid == 0) ends.own[c] = ends.spec[c] = ends.s32[c] = ends.s64[c] = xoff[c];
     return;
   }
   const int i0 = start[c], ni = count[c];
   if (damping > 0.0 && tid < ni) own[tid] = make_double4(x[i0 + tid], y[i0 + tid], z[i0 + tid], s[i0 + tid] * s[i0 + tid]);
-  if (tid < 2) n01[tid] = 0;
+  if (tid < XC_COUNT) num[tid] = 0;
   long long pos = xoff[c];
   for (int g0 = o0; g0 < o1; g0 += 256) {
-    const int B   = g0 + tid < o1 ? src[g0 + tid] : -1;
+    const int gn  = min(256, o1 - g0);
+    const int B   = tid < gn ? src[g0 + tid] : -1;
     const int nb  = B >= 0 ? count[B] : 0;
     int incl      = wave_scan_incl(nb, lane);
     __syncthreads();
@@ -641,9 +718,10 @@ __global__ __launch_bounds__(256) void k_xclass(const int* __restrict__ off, con
     __syncthreads();
     for (int q0 = 64 * wv; q0 < total; q0 += 256) {
       const int q = q0 + lane;
-      int j = 0, cl = 3;
+      int j = 0;
+      unsigned cl = XC_COUNT;
       if (q < total) {
-        int lo = 0, hi = min(256, o1 - g0);  // last leaf whose first entry is at or before q
+        int lo = 0, hi = gn;  // last leaf whose first entry is at or before q
         while (hi - lo > 1) {
           const int mid = (lo + hi) >> 1;
           if (pre[mid] <= q)
@@ -652,9 +730,9 @@ __global__ __launch_bounds__(256) void k_xclass(const int* __restrict__ off, con
             hi = mid;
         }
         j  = st[lo] + (q - pre[lo]);
-        cl = 0;
+        cl = j >= i0 && j < i0 + ni ? XC_OWN : XC_NEAR;
       }
-      const double sj = q < total && damping > 0.0 && (j < i0 || j >= i0 + ni) ? s[j] : 0.0;
+      const double sj = cl == XC_NEAR && damping > 0.0 ? s[j] : 0.0;
       double m        = 1e300;
       if (sj > 0.0) {
         const double xj = x[j], yj = y[j], zj = z[j];
@@ -666,41 +744,59 @@ __global__ __launch_bounds__(256) void k_xclass(const int* __restrict__ off, con
           if ((i & 7) == 7 && __all(m < stop)) break;  // (of the lanes still searching)
         }
         const double v = damping * sj * sqrt(m);
-        cl = v < kFarClass32 * (1.0 + 1e-9) ? 0 : (v < kTholeCutoff * (1.0 + 1e-9) ? 1 : 2);
+        cl = v < kFarClass32 * (1.0 + 1e-9) ? XC_NEAR : (v < kTholeCutoff * (1.0 + 1e-9) ? XC_MID : XC_FAR);
       }
-      if (q < total) ent[pos + q] = (unsigned)j | ((unsigned)cl << kXclsShift);
-      const int c0 = __popcll(__ballot(cl == 0)), c1 = __popcll(__ballot(cl == 1));
-      if (lane == 0) {
-        atomicAdd(&n01[0], c0);
-        atomicAdd(&n01[1], c1);
+      if (q < total) ent[pos + q] = (unsigned)j | (cl << kXclsShift);
+#pragma unroll
+      for (unsigned k : {XC_OWN, XC_NEAR, XC_MID}) {
+        const int n = __popcll(__ballot(cl == k));
+        if (lane == 0 && n) atomicAdd(&num[k], n);
       }
+    }
+    if (sk.off) {  // partners among this group's leaves (each entry moves to XC_PARTNER once)
+      __threadfence();
+      __syncthreads();
+      for (int i = i0 + tid; i < i0 + ni; i += 256)
+        for (int k = sk.off[i]; k < sk.off[i + 1]; ++k) {
+          const int e = (int)(sk.ent[k] & kSkipSite);
+          if (e >= i0 && e < i0 + ni) continue;
+          const int L = near_entry(off, src, c, leaf_of[e]) - g0;
+          if (L < 0 || L >= gn || src[g0 + L] != leaf_of[e]) continue;  // in another group, or not near
+          const unsigned was =
+              atomicMin(&ent[pos + pre[L] + (e - st[L])], (unsigned)e | ((unsigned)XC_PARTNER << kXclsShift));
+          if (was >> kXclsShift == XC_PARTNER) continue;
+          atomicAdd(&num[XC_PARTNER], 1);
+          atomicAdd(&num[was >> kXclsShift], -1);
+        }
     }
     pos += total;
   }
   __syncthreads();
   if (tid == 0) {
-    xs32[c] = xoff[c] + n01[0];
-    xs64[c] = xoff[c] + n01[0] + n01[1];
+    long long e  = xoff[c];
+    ends.own[c]  = e += num[XC_OWN];  // (a theta far above 1 can make a leaf far from itself: none)
+    ends.spec[c] = e += num[XC_PARTNER];
+    ends.s32[c]  = e += num[XC_NEAR];
+    ends.s64[c]  = e + num[XC_MID];
   }
 }
 
 // One wavefront per cell: its entries written class by class, each class in near-list order (one pass,
 // compaction with a ballot per class and 64 entries).
 __global__ __launch_bounds__(256) void k_xfill(int ncells, const unsigned* __restrict__ ent,
-                                               const long long* __restrict__ xoff, const long long* __restrict__ xs64,
-                                               const long long* __restrict__ xs32, int* __restrict__ xsrc) {
+                                               const long long* __restrict__ xoff, XEnds ends, int* __restrict__ xsrc) {
   const int c = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (c >= ncells) return;
   const unsigned long long below = (1ull << lane) - 1ull;
-  const long long e1 = xoff[c + 1];
-  long long pos[3]   = {xoff[c], xs32[c], xs64[c]};
-  for (long long e0 = pos[0]; e0 < e1; e0 += 64) {
-    const unsigned v = e0 + lane < e1 ? ent[e0 + lane] : 0xffffffffu;
+  const long long e0 = xoff[c], e1 = xoff[c + 1];
+  long long pos[XC_COUNT] = {e0, ends.own[c], ends.spec[c], ends.s32[c], ends.s64[c]};
+  for (long long e = e0; e < e1; e += 64) {
+    const unsigned v = e + lane < e1 ? ent[e + lane] : 0xffffffffu;
     const unsigned k = v >> kXclsShift;
 #pragma unroll
-    for (unsigned cl = 0; cl < 3; ++cl) {
+    for (unsigned cl = 0; cl < XC_COUNT; ++cl) {
       const unsigned long long m = __ballot(k == cl);
-      if (k == cl) xsrc[pos[cl] + __popcll(m & below)] = (int)(v & ((1u << kXclsShift) - 1u));
+      if (k == cl) xsrc[pos[cl] + __popcll(m & below)] = (int)(v & kXclsSite);
       pos[cl] += __popcll(m);
     }
   }
@@ -724,46 +820,43 @@ void build_near_expanded(System& S) {
   CPPE_HIP_CHECK(hipMemcpyAsync(&total, T.xoff.p + nc, sizeof(long long), hipMemcpyDeviceToHost, st));
   CPPE_HIP_CHECK(hipStreamSynchronize(st));
   T.xsrc.alloc(std::max<long long>(total, 1));
+  T.xspec.alloc(nc);
   T.xsplit[0].alloc(nc);
   T.xsplit[1].alloc(nc);
-  // (site indices below 2^30: a system of more sites has no room for its lists on the device)
+  build_pair_skips(S);
+  dbuf<long long> xown;
+  xown.alloc(nc);
+  const XEnds ends{xown.p, T.xspec.p, T.xsplit[1].p, T.xsplit[0].p};
+  // (site indices below 2^29: a system of more sites has no room for its lists on the device)
   dbuf<unsigned> ent;
   ent.alloc(std::max<long long>(total, 1));
-  hipLaunchKernelGGL(k_xclass, dim3(nc), dim3(256), 0, st, T.p2p_off.p, T.p2p_src.p, T.start.p, T.count.p, S.x.p,
-                     S.y.p, S.z.p, S.s.p, S.s.p ? S.opts.damping : 0.0, T.xoff.p, ent.p, T.xsplit[0].p, T.xsplit[1].p);
-  hipLaunchKernelGGL(k_xfill, dim3(ceil_div(nc, 4)), dim3(256), 0, st, nc, ent.p, T.xoff.p, T.xsplit[0].p,
-                     T.xsplit[1].p, T.xsrc.p);
+  hipLaunchKernelGGL(k_xclass, dim3(nc), dim3(256), 0, st, T.p2p_off.p, T.p2p_src.p, T.start.p, T.count.p, T.leaf_of.p,
+                     S.x.p, S.y.p, S.z.p, S.s.p, S.s.p ? S.opts.damping : 0.0, S.skips.lists(), T.xoff.p, ent.p, ends);
+  hipLaunchKernelGGL(k_xfill, dim3(ceil_div(nc, 4)), dim3(256), 0, st, nc, ent.p, T.xoff.p, ends, T.xsrc.p);
   CPPE_HIP_CHECK(hipStreamSynchronize(st));
   T.nx    = total;
   T.xdamp = S.opts.damping;
 }
 
 // ---- lists of the symmetric near field (near_sym.hh) -------------------------------------------
-// Entry of leaf A in the near list of leaf B (sorted by source leaf); without one, where it would stand.
-__device__ __forceinline__ int near_entry(const int* __restrict__ off, const int* __restrict__ src, int B, int A) {
-  int lo = off[B], hi = off[B + 1];
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (src[mid] < A)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo;
-}
-
-// One wavefront per cell, lanes over its near list: *one_sided set if a leaf near it does not have it as near leaf.
-__global__ __launch_bounds__(256) void k_near_one_sided(int ncells, const int* __restrict__ off,
-                                                        const int* __restrict__ src, int* __restrict__ one_sided) {
+// One wavefront per cell, lanes over its near list: *one_sided set if a leaf near it does not have it as near
+// leaf, or if it is a leaf that is not near itself.
+__global__ __launch_bounds__(256) void k_near_one_sided(int ncells, const int* __restrict__ nchild,
+                                                        const int* __restrict__ off, const int* __restrict__ src,
+                                                        int* __restrict__ one_sided) {
   const int A = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (A >= ncells) return;
+  if (nchild[A] == 0) {
+    const int e = near_entry(off, src, A, A);
+    if (e == off[A + 1] || src[e] != A) *one_sided = 1;
+  }
   for (int k = off[A] + (threadIdx.x & 63); k < off[A + 1]; k += 64) {
     const int B = src[k], e = near_entry(off, src, B, A);
     if (e == off[B + 1] || src[e] != A) *one_sided = 1;
   }
 }
 
-// Whether B near A always comes with A near B. The walk splits the target first in a pair of equal cells, so at a
+// Whether B near A always comes with A near B, and every leaf is near itself. The walk splits the target first in a pair of equal cells, so at a
 // theta where a cell touches the acceptance bound it may take a pair as far from one side only (at theta = 1
 // 69 of the 84,595 near pairs of 60,000 sites).
 bool near_lists_symmetric(System& S) {
@@ -773,8 +866,8 @@ bool near_lists_symmetric(System& S) {
     one_sided.alloc(1);
     int h = 0;
     CPPE_HIP_CHECK(hipMemcpyAsync(one_sided.p, &h, sizeof(int), hipMemcpyHostToDevice, S.stream));
-    hipLaunchKernelGGL(k_near_one_sided, dim3(ceil_div(T.ncells, 4)), dim3(256), 0, S.stream, T.ncells, T.p2p_off.p,
-                       T.p2p_src.p, one_sided.p);
+    hipLaunchKernelGGL(k_near_one_sided, dim3(ceil_div(T.ncells, 4)), dim3(256), 0, S.stream, T.ncells, T.nchild.p,
+                       T.p2p_off.p, T.p2p_src.p, one_sided.p);
     CPPE_HIP_CHECK(hipMemcpyAsync(&h, one_sided.p, sizeof(int), hipMemcpyDeviceToHost, S.stream));
     CPPE_HIP_CHECK(hipStreamSynchronize(S.stream));
     T.near_symmetric = h == 0;

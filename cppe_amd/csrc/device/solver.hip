@@ -741,9 +741,9 @@ __global__ __launch_bounds__(T) void k_cg_tiny(TinyArgs a) {
       if (i < n && j < n && !(skip >> q & 1u)) {
         const double dx = xi - pos[0][j], dy = yi - pos[1][j], dz = zi - pos[2][j];
         if (a.damping > 0.0)
-          geo_m1_f64<true, true>(dx, dy, dz, di * pos[3][j], c3[q], cf[q]);
+          geo_m1_f64<true>(dx, dy, dz, di * pos[3][j], c3[q], cf[q]);
         else
-          geo_m1_f64<false, true>(dx, dy, dz, 0.0, c3[q], cf[q]);
+          geo_m1_f64<false>(dx, dy, dz, 0.0, c3[q], cf[q]);
       }
     }
   }

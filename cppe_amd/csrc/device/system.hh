@@ -10,6 +10,21 @@
 
 namespace cppe_dev {
 
+// Skip lists of the sites (build_pair_skips): entries off[i] .. off[i + 1] of site i name the partners whose
+// pairs with it the near fields leave out; null without exclusions.
+constexpr unsigned kSkipKeep = 1u << 31;         // only the partner excludes the pair: the field at site i keeps it
+constexpr unsigned kSkipSite = (1u << 30) - 1u;  // the partner
+struct SkipLists {
+  const int* off;
+  const unsigned* ent;
+};
+struct PairSkips {
+  dbuf<int> off;
+  dbuf<unsigned> ent;
+  bool built = false, one_way = false;  // one_way: an entry is marked kSkipKeep
+  SkipLists lists() const { return SkipLists{built ? off.p : nullptr, ent.p}; }
+};
+
 // Lists of the symmetric near-field kernel (near_sym.hh) for chunks of ts targets: the work items;
 // per leaf A its upper list (A's own sites, then the sites of its near leaves B > A; FP32: in the
 // class order of the expanded near list, FP64: in near-list order), with the reverse slot of each entry (for chunk 0 and component x, and
@@ -45,11 +60,13 @@ struct Octree {
   long long nx = -1;           // total length (-1: not built)
   dbuf<long long> xoff;        // ncells+1 offsets
   dbuf<int> xsrc;              // source sites (device order)
-  // Each leaf's expanded list is ordered by the smallest Thole argument v of each source over the
-  // leaf's targets: v_min < 18, then 18 <= v_min < 40, then v_min >= 40 (stable within each class).
+  // Each leaf's expanded list begins with its own sites and the sites that their skip lists name in other leaves (up
+  // to xspec: the only entries that can be a target itself or a pair left out); the rest is ordered by the
+  // smallest Thole argument v of each source over the leaf's targets: v_min < 18, then 18 <= v_min < 40,
+  // then v_min >= 40 (each class in near-list order).
   // xsplit[1] (FP32) / xsplit[0] (FP64): offset of the first source that takes the undamped pair
   // in that precision for every target of the leaf (kFarClass32, kTholeCutoff).
-  dbuf<long long> xsplit[2];
+  dbuf<long long> xspec, xsplit[2];
   double xdamp = 0.0;  // damping factor of the classification (valid for kernels with damping >= xdamp)
   SymLists sym[2][5];  // symmetric near field (FP64, FP32) with chunks of 4, 6, 8, 12, 16 targets (sym_slot)
   int near_symmetric = -1;  // near_lists_symmetric's answer (-1: not asked yet)
@@ -157,6 +174,7 @@ struct System {
     return h;
   }
   std::vector<int> h_excl_off, h_excl_idx;  // caller order, values as given
+  PairSkips skips;
 
   Octree tree;
   FmmState* fmm = nullptr;
@@ -217,6 +235,7 @@ void build_octree(System& S, const double* pos);
 void device_scan(System& S, const int* in, int* out, int n);
 void build_lists(System& S);
 void build_near_expanded(System& S);
+void build_pair_skips(System& S);
 bool near_lists_symmetric(System& S);
 // lists of the symmetric near-field kernel with chunks of ts targets (4, 6, 8, 12 or 16) into
 // S.tree.sym[prec][sym_slot(ts)] (prec: 0 FP64, 1 FP32)
