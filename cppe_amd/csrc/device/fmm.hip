@@ -38,7 +38,8 @@ constexpr int kOverlapSites = 1536;
 // cppe_hip_set_tune): what a program that only builds a system and solves runs with.
 static FmmTune default_tune(System& S) {
   FmmTune t;
-  const Octree& T = S.tree;
+  const Octree& T     = S.tree;
+  t.own_displacements = true;
   t.near_block[0] = t.near_block[1] = 128;
   if (one_leaf_system(S)) {
     // Direct summation: the tiled symmetric form, whose reverse blocks take 3 n^2 / (2 TB) values;
@@ -52,9 +53,9 @@ static FmmTune default_tune(System& S) {
     t.near_variant[1] = fits(kSymTs[1][k], sizeof(float)) ? 9 + k : 8;
     return t;
   }
-  // Trees: lanes as sources. FP32: chunks of 16 targets once they alone make enough wavefronts, else 8.
-  t.near_variant[1] = std::max(T.nleaves, S.n / 16) >= kLanesWide ? 7 : 8;
-  t.near_block[1]   = t.near_variant[1] == 7 ? 128 : 256;
+  // Trees: lanes as sources. FP32: chunks of 8 targets (16 positions of 64 bits do not fit the scalar registers).
+  t.near_variant[1] = 8;
+  t.near_block[1]   = 256;
   // FP64: chunks of 4; the symmetric form for the plain form's solves of larger systems with small
   // leaves, where sharing a pair's geometry outweighs the reverse blocks (a mixed solve runs one or
   // two FP64 applies, which would not pay for its lists). Its reverse slots are 32-bit indices: at
@@ -298,7 +299,7 @@ void fmm_reserve(System& S, bool mixed, int nrhs) {
     if (v == 4) ensure_clusters(S);
     if (near_sym_variant(v)) {
       if (one_leaf_system(S))
-        ensure_dsym(S, prec, kSymTs[prec][v - 9], S.opts.damping);
+        ensure_dsym(S, prec, kSymTs[prec][v - 9]);
       else
         ensure_sym(S, prec, kSymTs[prec][v - 9], S.opts.damping);
     } else if (v == 3 || v >= 5) {
@@ -373,6 +374,7 @@ void fmm_autotune(System& S, int reps, int* choice, double* ms) {
   FmmState& F = state(S);
   F.tune      = default_tune(S);  // (an earlier choice may be one that this tree does not allow)
   fmm_reserve(S, true, 1);
+  F.tune.own_displacements = false;
   hipStream_t st = S.stream;
   hipEvent_t ev[8];
   for (auto& e : ev) CPPE_HIP_CHECK(hipEventCreate(&e));
@@ -468,6 +470,7 @@ void fmm_autotune(System& S, int reps, int* choice, double* ms) {
 
 void fmm_set_tune(System& S, const int* choice) {
   FmmState& F = state(S);
+  F.tune.own_displacements = false;
   for (int prec = 0; prec < 2; ++prec) {
     F.tune.near_variant[prec] = choice[4 * prec];
     F.tune.near_block[prec]   = choice[4 * prec + 1];

@@ -48,6 +48,8 @@ struct FmmTune {
   int overlap[2]      = {0, 0};    // far field on a second stream beside the near field (staged variants):
                                    // 0 none, 1 the whole far field, 2 M2L / L2L after the upward pass,
                                    // 3 the whole far field enqueued ahead of the near field
+  bool own_displacements = false;  // FP32 pairs of the symmetric direct form and of variant 8: displacements formed in
+                                   // FP64 (untuned systems: as the thread-per-target form, whose place they take)
   int near_splits[2]  = {1, 1};    // overlapped forms: the near field in 1, 2 or 4 launches, so the
                                    // far field's kernels get the device between them
 };
@@ -985,22 +987,22 @@ struct alignas(K == 1 ? 4 * sizeof(R) : 16) StagedRec {  // K = 1: two 16-byte (
 // a then carries the factor log2(e). FAR: a source past the precision's far class for every target of the leaf (never
 // the target itself or a skipped pair): the undamped geometry (FP32: from v >= 18 on, where the screening it
 // leaves out moves the field by less than the FP32 rounding; FP64: from v >= 40 on, where it is exactly 1).
-// SELF0: a pair without displacement (the site itself, where the kernel takes it in) is zero; skip: this pair is.
+// SELF0: a pair without displacement (the site itself, where the kernel takes it in) is zero; keep: pairs.hh.
 template <typename R, bool DAMP, bool B2, bool FAR, bool SELF0>
-__device__ __forceinline__ void staged_geo(R dx, R dy, R dz, R a, R& c3, R& cf, bool skip = false) {
+__device__ __forceinline__ void staged_geo(R dx, R dy, R dz, R a, R& c3, R& cf, int keep = -1) {
   if constexpr (sizeof(R) == 8)
-    geo_m1_f64<DAMP && !FAR, SELF0 && !FAR>(dx, dy, dz, a, c3, cf, skip);
+    geo_m1_f64<DAMP && !FAR, SELF0 && !FAR>(dx, dy, dz, a, c3, cf, keep);
   else if constexpr (FAR)
     geo_m1_f32<false, false>(dx, dy, dz, a, c3, cf);
   else if constexpr (B2)
-    geo_m1_f32_b2<SELF0>(dx, dy, dz, a, c3, cf, skip);
+    geo_m1_f32_b2<SELF0>(dx, dy, dz, a, c3, cf, keep);
   else
-    geo_m1_f32<DAMP, SELF0>(dx, dy, dz, a, c3, cf, skip);
+    geo_m1_f32<DAMP, SELF0>(dx, dy, dz, a, c3, cf, keep);
 }
 
 // one pair against the K dipoles of a staged record, given its displacement; f holds 3 K accumulators
 template <typename R, bool DAMP, bool B2, int K, bool FAR = false, bool SELF0 = true>
-__device__ __forceinline__ void staged_pair(R dx, R dy, R dz, R di, const StagedRec<R, K>& r, R* f, bool skip = false) {
+__device__ __forceinline__ void staged_pair(R dx, R dy, R dz, R di, const StagedRec<R, K>& r, R* f, int keep = -1) {
   if constexpr (FAR && sizeof(R) == 4) {
     float ri3, m3;
     geo_far_f32(dx, dy, dz, ri3, m3);
@@ -1010,7 +1012,7 @@ __device__ __forceinline__ void staged_pair(R dx, R dy, R dz, R di, const Staged
                   f[3 * k + 2]);
   } else {
     R c3, cf;
-    staged_geo<R, DAMP, B2, FAR, SELF0>(dx, dy, dz, di * r.s, c3, cf, skip);
+    staged_geo<R, DAMP, B2, FAR, SELF0>(dx, dy, dz, di * r.s, c3, cf, keep);
 #pragma unroll
     for (int k = 0; k < K; ++k)
       acc_m1(c3, cf, dx, dy, dz, r.m[3 * k], r.m[3 * k + 1], r.m[3 * k + 2], f[3 * k], f[3 * k + 1], f[3 * k + 2]);
@@ -1371,45 +1373,60 @@ __global__ __launch_bounds__(256) void k_fmm_skip_fix(NearArgs a, SkipLists sk, 
 }
 
 // Skip list entries of a work item's targets i0 .. i0 + T - 1 and, for a stage of 64 sources, one per lane, which
-// targets leave the lane's source out. The first 64 entries stand in wavefront-private LDS, each with the target it
-// belongs to (in registers they would cost the tiled direct form its second block on a CU); any beyond are read
-// from memory, one after another. A kernel keeps what it needs to tell which of them can meet a stage (its lane's).
+// targets leave the lane's source out (bit t: target t). A lane holds one of the first 64 entries with its target;
+// entries beyond are read from memory, one after another. OWN: entries marked kSkipKeep do not count. mem: 64
+// words of wavefront-private LDS.
 struct ItemSkips {
-  const int2* lds;
   SkipLists sk;
-  int i0, off = 0, n = 0;
-  // this lane's entry goes to ent (lane < n)
-  __device__ __forceinline__ ItemSkips(const SkipLists& s, int i0_, int T, int lane, int2* mem, unsigned& ent)
-      : lds(mem), sk(s), i0(i0_) {
-    ent = 0;
+  int* mem;
+  int i0, lane, off = 0, n = 0;
+  unsigned ent = kSkipSite;  // this lane's entry (no site: none)
+  int tgt      = 0;          // its target
+  __device__ __forceinline__ ItemSkips(const SkipLists& s, int i0_, int T, int lane_, int* mem_)
+      : sk(s), mem(mem_), i0(i0_), lane(lane_) {
     if (!sk.off || T <= 0) return;
-    off = __builtin_amdgcn_readfirstlane(sk.off[i0]);
-    n   = __builtin_amdgcn_readfirstlane(sk.off[i0 + T]) - off;
-    if (lane < n) {
-      int t = 0;
-      ent   = sk.ent[off + lane];
-      while (sk.off[i0 + t + 1] - off <= lane) ++t;
-      mem[lane] = make_int2((int)ent, t);
-    }
-    wave_lds_barrier();
+    const int o = sk.off[i0 + min(lane, T)];  // lane t: where the entries of target t begin
+    off         = __builtin_amdgcn_readlane(o, 0);
+    n           = __builtin_amdgcn_readlane(o, T) - off;
+    if (lane < n) ent = sk.ent[off + lane];
+    for (int u = 1; u < T; ++u) tgt += __builtin_amdgcn_readlane(o, u) - off <= lane;
   }
-  // Bit t of the result: target t skips site j, by the entries of lanes m (and all beyond 64). OWN: entries
-  // marked kSkipKeep do not count.
+  __device__ __forceinline__ int site() const { return (int)(ent & kSkipSite); }
+  // lane l's source is site first + l, by the first 64 entries; ok: this lane's entry can be one of them
+  template <bool OWN>
+  __device__ __forceinline__ unsigned run(int first, bool ok) const {
+    unsigned skip = 0;
+    const bool in = ok && (unsigned)(site() - first) < 64u && !(OWN && (ent & kSkipKeep));
+    if (__ballot(in) != 0) {
+      mem[lane] = 0;
+      wave_lds_barrier();
+      if (in) atomicOr(&mem[site() - first], 1 << tgt);
+      wave_lds_barrier();
+      skip = (unsigned)mem[lane];
+    }
+    return skip;
+  }
+  // the lane's source is site j, by the entries of lanes m
   template <bool OWN>
   __device__ __forceinline__ unsigned of(int j, unsigned long long m) const {
     unsigned skip = 0;
-    auto take     = [&](unsigned v, int t) {
-      if ((int)(v & kSkipSite) == j && !(OWN && (v & kSkipKeep))) skip |= 1u << t;
-    };
     while (m) {
-      const int2 v = lds[__ffsll(m) - 1];
+      const int p      = __ffsll(m) - 1;
+      const unsigned v = (unsigned)__builtin_amdgcn_readlane((int)ent, p);
       m &= m - 1;
-      take((unsigned)v.x, v.y);
+      if ((int)(v & kSkipSite) == j && !(OWN && (v & kSkipKeep))) skip |= 1u << __builtin_amdgcn_readlane(tgt, p);
     }
-    int t = 0;
+    return skip;
+  }
+  // the lane's source is site j, by the entries beyond
+  template <bool OWN>
+  __device__ __forceinline__ unsigned rest(int j) const {
+    unsigned skip = 0;
+    int t         = 0;
     for (int k = 64; k < n; ++k) {
       while (sk.off[i0 + t + 1] - off <= k) ++t;
-      take(sk.ent[off + k], t);
+      const unsigned v = sk.ent[off + k];
+      if ((int)(v & kSkipSite) == j && !(OWN && (v & kSkipKeep))) skip |= 1u << t;
     }
     return skip;
   }
@@ -1813,10 +1830,10 @@ inline long long dsym_segment(int n, int tb) {
 
 // Items and blocks of the symmetric direct summation with TS targets per wavefront (systems whose
 // tree is one leaf); built on the host once per chunk size.
-inline FmmState::DSym& ensure_dsym(System& S, int prec, int ts, double damping) {
+inline FmmState::DSym& ensure_dsym(System& S, int prec, int ts) {
   FmmState& F       = *S.fmm;
   FmmState::DSym& D = F.dsym[prec];
-  ensure_sym_trec(S, prec, damping);
+  ensure_pos4(S);
   build_pair_skips(S);
   if (D.ts != ts) {
     const int n = S.n, TB = kDSymW * ts;
@@ -1874,10 +1891,6 @@ constexpr double kDSymDefaultBytes = 4.0e9;
 // Sites from which an untuned direct-summation system takes FP32 chunks of 12 targets instead of 8
 // (apply at 9,000 sites 102 us either way, at 24,000 397 against 421 us, at 60,000 2.05 against 2.17 ms).
 constexpr int kDSym32Wide = 16384;
-// Leaves (or sixteenths of the sites) from which an untuned tree's FP32 near field takes chunks of 16
-// targets: mixed solves with 16 / 8 took 1.65 / 1.55 ms at 12,000 sites, 3.36 / 3.30 at 60,000, 7.64 / 7.65 at
-// 120,000 (8,200 chunks of 16) and 12.0 / 12.3 at 300,000 (30,000 chunks).
-constexpr int kLanesWide = 16384;
 // Sites and mean leaf size for which an untuned plain-form tree takes the symmetric near field: FP64
 // solves with it / with lanes as sources took 3.3 / 2.6 ms at 12,000 sites (23 a leaf), 7.7 / 8.2 at 60,000 (15
 // a leaf), 24.0 / 23.9 at 120,000 (29 a leaf) and 34.4 / 35.6 at 300,000 (10 a leaf).
@@ -1895,7 +1908,7 @@ void launch_direct_sym(System& S, const NearArgs& a, const MU4* mu4, const R* L,
   FmmState& F        = *S.fmm;
   const Octree& T    = S.tree;
   constexpr int prec = sizeof(R) == 4;
-  FmmState::DSym& D  = ensure_dsym(S, prec, TS, a.damping);
+  FmmState::DSym& D  = ensure_dsym(S, prec, TS);
   constexpr bool kB2 = prec && DAMP;
   const bool b2      = kB2 && S.all_damped;
   hipStream_t st     = S.stream;
@@ -1909,18 +1922,20 @@ void launch_direct_sym(System& S, const NearArgs& a, const MU4* mu4, const R* L,
     rev = F.drev64.p;
   }
   if (S.prof) CPPE_HIP_CHECK(hipEventRecord(S.prof[6], st));
-  const dim3 g(D.nitems), b(64 * kDSymW);
-  if constexpr (prec) {
+  auto go = [&](auto pos, auto bb) {
+    hipLaunchKernelGGL((k_direct_sym<R, decltype(pos), DAMP, decltype(bb)::value, TS, kDSymW, MU4>), dim3(D.nitems),
+                       dim3(64 * kDSymW), 0, st, a, da, mu4, fwd, rev);
+  };
+  auto go_b = [&](auto pos) {
     if (b2)
-      hipLaunchKernelGGL((k_direct_sym<R, DAMP, kB2, TS, kDSymW, MU4, float4>), g, b, 0, st, a, da, F.sym_t32.p, mu4,
-                         fwd, rev);
+      go(pos, std::integral_constant<bool, kB2>{});
     else
-      hipLaunchKernelGGL((k_direct_sym<R, DAMP, false, TS, kDSymW, MU4, float4>), g, b, 0, st, a, da, F.sym_t32.p,
-                         mu4, fwd, rev);
-  } else {
-    hipLaunchKernelGGL((k_direct_sym<R, DAMP, false, TS, kDSymW, MU4, double4>), g, b, 0, st, a, da, F.sym_t64.p,
-                       mu4, fwd, rev);
-  }
+      go(pos, std::false_type{});
+  };
+  if (prec && !F.tune.own_displacements)
+    go_b(R{});
+  else
+    go_b(double{});
   if (S.prof) CPPE_HIP_CHECK(hipEventRecord(S.prof[7], st));
   // the gather ends the apply: alpha^-1 mu and, when the CG step asked, its partials
   const bool more = with_l2p || S.skips.one_way;
@@ -2019,10 +2034,11 @@ void launch_near(System& S, const NearArgs& a, const MU4* mu4, const R* L, bool 
     const Octree& T = S.tree;
     constexpr bool kB2 = sizeof(R) == 4 && DAMP;  // the branch-free FP32 pair needs every site damped
     const bool b2      = kB2 && S.all_damped;
+    const bool own      = prec && F.tune.own_displacements;  // (untuned systems: variant 8)
     // far-source stages: valid for damping factors at least the classification's
-    const long long* xs = (DAMP && a.damping >= T.xdamp) ? T.xsplit[prec].p : nullptr;
+    const long long* xs = (DAMP && a.damping >= T.xdamp) ? T.xsplit[own ? 2 : prec].p : nullptr;
     const int splits    = with_l2p ? 1 : std::max(1, F.tune.near_splits[prec]);  // (see the staged variants)
-    auto go = [&](auto l2p, auto ts, auto bb) {
+    auto go = [&](auto pos, auto l2p, auto ts, auto bb) {
       constexpr int TS = decltype(ts)::value;
       const int ni     = ensure_near_chunks(S, TS);
       const int4* items = F.near_chunks[lanes_slot(TS)].p;
@@ -2030,23 +2046,27 @@ void launch_near(System& S, const NearArgs& a, const MU4* mu4, const R* L, bool 
       for (int k = 0; k < splits; ++k) {
         const int c0 = (int)((long long)ni * k / splits), c1 = (int)((long long)ni * (k + 1) / splits);
         if (c1 <= c0) continue;
-        hipLaunchKernelGGL((k_fmm_near_ls<P, R, DAMP, MODE, MU4, decltype(l2p)::value, TS, decltype(bb)::value, K>),
-                           dim3(ceil_div(c1 - c0, block / 64)), dim3(block), 0, st, a, S.skips.lists(), items + c0, c1 - c0,
-                           T.xoff.p, T.xsrc.p, T.xspec.p, xs, mu4, L, lstride);
+        const LanesArgs<R, MU4> la{a,        S.skips.lists(), items + c0, c1 - c0, T.xoff.p, T.xsrc.p,
+                                   T.xspec.p, xs,              mu4,        L,       lstride};
+        hipLaunchKernelGGL((k_fmm_near_ls<P, R, decltype(pos), DAMP, MODE, MU4, decltype(l2p)::value, TS,
+                                          decltype(bb)::value, K>),
+                           dim3(ceil_div(c1 - c0, block / 64)), dim3(block), kLanesLds<R> * (block / 64), st, la);
       }
       if (S.prof) CPPE_HIP_CHECK(hipEventRecord(S.prof[7], st));
     };
-    auto go_b = [&](auto l2p, auto ts) {
+    auto go_b = [&](auto pos, auto l2p, auto ts) {
       if (b2)
-        go(l2p, ts, std::integral_constant<bool, kB2>{});
+        go(pos, l2p, ts, std::integral_constant<bool, kB2>{});
       else
-        go(l2p, ts, std::false_type{});
+        go(pos, l2p, ts, std::false_type{});
     };
     auto go_ts = [&](auto l2p) {
       if (var == 7)
-        go_b(l2p, std::integral_constant<int, near_lanes_ts(7, kPrec, K)>{});
+        go_b(R{}, l2p, std::integral_constant<int, near_lanes_ts(7, kPrec, K)>{});
+      else if (own)
+        go_b(double{}, l2p, std::integral_constant<int, near_lanes_ts(8, kPrec, K)>{});
       else
-        go_b(l2p, std::integral_constant<int, near_lanes_ts(8, kPrec, K)>{});
+        go_b(R{}, l2p, std::integral_constant<int, near_lanes_ts(8, kPrec, K)>{});
     };
     if (with_l2p)
       go_ts(std::true_type{});

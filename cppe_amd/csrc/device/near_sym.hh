@@ -41,18 +41,21 @@ template <typename R>
 struct alignas(4 * sizeof(R)) SymVec4 {
   R x, y, z, w;
 };
-// a target of a work item: position (FP32: offset from the leaf centre) and damping rate; dipole
-template <typename R>
+// a target of a work item: position and damping rate; dipole. POS: the type positions are held and subtracted in, as in
+// the lanes form (near_lanes.hh): double absolute positions, float offsets from the leaf's centre.
+template <typename R, typename POS>
 struct SymTarget {
-  SymVec4<R> p, m;
+  POS x, y, z;
+  R w;
+  SymVec4<R> m;
 };
 
-// Geometry once, field at both ends: f += T(d) mu_s, r += T(d) mu_t (skip: neither).
-template <typename R, bool DAMP, bool B2, bool FAR>
-__device__ __forceinline__ void sym_pair(const SymTarget<R>& t, R xs, R ys, R zs, R ss, R mxs, R mys, R mzs, R& fx,
-                                         R& fy, R& fz, R& rx, R& ry, R& rz, bool skip) {
-  const SymVec4<R> tp = t.p, tm = t.m;
-  const R dx = tp.x - xs, dy = tp.y - ys, dz = tp.z - zs;
+// Geometry once, field at both ends: f += T(d) mu_s, r += T(d) mu_t (keep: pairs.hh).
+template <typename R, bool DAMP, bool B2, bool FAR, typename POS>
+__device__ __forceinline__ void sym_pair(const SymTarget<R, POS>& t, POS xs, POS ys, POS zs, R ss, R mxs, R mys, R mzs, R& fx,
+                                         R& fy, R& fz, R& rx, R& ry, R& rz, int keep) {
+  const SymVec4<R> tm = t.m;
+  const R dx = (R)(t.x - xs), dy = (R)(t.y - ys), dz = (R)(t.z - zs);
   if constexpr (FAR && sizeof(R) == 4) {
     float ri3, m3;
     geo_far_f32(dx, dy, dz, ri3, m3);
@@ -60,7 +63,7 @@ __device__ __forceinline__ void sym_pair(const SymTarget<R>& t, R xs, R ys, R zs
     acc_far_f32(ri3, m3, dx, dy, dz, tm.x, tm.y, tm.z, rx, ry, rz);
   } else {
     R c3, cf;
-    staged_geo<R, DAMP, B2, FAR, false>(dx, dy, dz, tp.w * ss, c3, cf, skip);
+    staged_geo<R, DAMP, B2, FAR, false>(dx, dy, dz, t.w * ss, c3, cf, keep);
     acc_m1(c3, cf, dx, dy, dz, mxs, mys, mzs, fx, fy, fz);
     acc_m1(c3, cf, dx, dy, dz, tm.x, tm.y, tm.z, rx, ry, rz);
   }
@@ -127,23 +130,19 @@ __global__ __launch_bounds__(256) void k_fmm_near_sym(NearArgs a, SymArgs b, con
   };
   // the item's targets in wavefront-private LDS (record, dipole), read with uniform addresses
   // (broadcast) inside the pair loops
-  __shared__ SymTarget<R> tl[4][TS];
-  SymTarget<R>* tg = tl[threadIdx.x >> 6];
+  __shared__ SymTarget<R, R> tl[4][TS];
+  SymTarget<R, R>* tg = tl[threadIdx.x >> 6];
   if (lane < T) {
     const TREC tr = trec[i0 + lane];
     const MU4 mt  = mu4[i0 + lane];
-    tg[lane].p    = SymVec4<R>{(R)tr.x, (R)tr.y, (R)tr.z, (R)tr.w};
-    tg[lane].m    = SymVec4<R>{(R)mt.x, (R)mt.y, (R)mt.z, R(0)};
+    tg[lane] = SymTarget<R, R>{(R)tr.x, (R)tr.y, (R)tr.z, (R)tr.w, {(R)mt.x, (R)mt.y, (R)mt.z, R(0)}};
   }
   wave_lds_barrier();
-  // skip list entries of the item's targets: partners in the leaf stand at e0 + (site - start); of the others only
-  // those in leaves above A are sources here
-  __shared__ int2 mem[4][64];
-  unsigned ent;
-  const ItemSkips its(b.sk, i0, T, lane, mem[threadIdx.x >> 6], ent);
-  const int partner              = (int)(ent & kSkipSite), at = partner - a.start[A];
-  const bool inside              = lane < its.n && (unsigned)at < (unsigned)a.count[A];
-  const unsigned long long above = __ballot(lane < its.n && !inside && a.leaf_of[partner] > A);
+  // skip list entries of the item's targets: own sites, and of the others those in leaves above A
+  __shared__ int mem[4][64];
+  const ItemSkips its(b.sk, i0, T, lane, mem[threadIdx.x >> 6]);
+  const bool inside              = (unsigned)(its.site() - a.start[A]) < (unsigned)a.count[A];
+  const unsigned long long above = __ballot(lane < its.n && !inside && a.leaf_of[its.site()] > A);
   // A's own sites: ordered pairs, field at the item's targets only
   for (long long q0 = e0; q0 < es; q0 += 64) {
     const bool act = q0 + lane < es;
@@ -152,14 +151,13 @@ __global__ __launch_bounds__(256) void k_fmm_near_sym(NearArgs a, SymArgs b, con
     convert(act ? a.pos4[j] : make_double4(0.0, 0.0, 0.0, 0.0), act ? mu4[j] : MU4{}, act, xs, ys, zs, ss, mx, my,
             mz);
     unsigned skip = (unsigned)(j - i0) < (unsigned)T ? 1u << (j - i0) : 0u;
-    skip |= its.template of<false>(j, __ballot(inside && (unsigned)(at - (int)(q0 - e0)) < 64u));
+    skip |= its.template run<false>(j - lane, inside) | its.template rest<false>(j);
 #pragma unroll
     for (int t = 0; t < TS; ++t) {
       if (t < T) {
-        const SymVec4<R> tp = tg[t].p;
-        const R dx = tp.x - xs, dy = tp.y - ys, dz = tp.z - zs;
+        const R dx = tg[t].x - xs, dy = tg[t].y - ys, dz = tg[t].z - zs;
         R c3, cf;
-        staged_geo<R, DAMP, B2, false, false>(dx, dy, dz, tp.w * ss, c3, cf, skip >> t & 1u);
+        staged_geo<R, DAMP, B2, false, false>(dx, dy, dz, tg[t].w * ss, c3, cf, keep_unless(skip, t));
         acc_m1(c3, cf, dx, dy, dz, mx, my, mz, f[t][0], f[t][1], f[t][2]);
       }
     }
@@ -185,8 +183,7 @@ __global__ __launch_bounds__(256) void k_fmm_near_sym(NearArgs a, SymArgs b, con
     R xs, ys, zs, ss, mx, my, mz;
     convert(pn, mn, act, xs, ys, zs, ss, mx, my, mz);
     const int2 dd = dn;
-    unsigned skip = 0;
-    if (above != 0 || its.n > 64) skip = its.template of<false>(jn, above);
+    const unsigned skip = its.template of<false>(jn, above) | its.template rest<false>(jn);
     if (q0 + 64 + lane < e1) {  // stage s + 1
       jn = jnn;
       pn = a.pos4[jnn];
@@ -201,13 +198,13 @@ __global__ __launch_bounds__(256) void k_fmm_near_sym(NearArgs a, SymArgs b, con
     if (q0 >= ef) {  // every pair of the stage beyond the precision's damping cutoff (uniform)
 #pragma unroll
       for (int t = 0; t < TS; ++t)
-        if (t < T) sym_pair<R, DAMP, B2, true>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz, false);
+        if (t < T) sym_pair<R, DAMP, B2, true>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz, -1);
     } else {
 #pragma unroll
       for (int t = 0; t < TS; ++t)
         if (t < T)
           sym_pair<R, DAMP, B2, false>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz,
-                                       skip >> t & 1u);
+                                       keep_unless(skip, t));
     }
     if (act) {
       const int o = dd.x + q * 3 * dd.y;
@@ -299,64 +296,61 @@ __device__ __forceinline__ long long dsym_rev_block(int J, int I, int TB) {
   return 3ll * TB * ((long long)J * (J - 1) / 2 + I);
 }
 
-template <typename R, bool DAMP, bool B2, int TS, int W, typename MU4, typename TREC>
-__global__ __launch_bounds__(64 * W) void k_direct_sym(NearArgs a, DSymArgs b, const TREC* __restrict__ trec,
-                                                       const MU4* __restrict__ mu4, R* __restrict__ fwd,
-                                                       R* __restrict__ rev) {
+template <typename R, typename POS, bool DAMP, bool B2, int TS, int W, typename MU4>
+__global__ __launch_bounds__(64 * W) void k_direct_sym(NearArgs a, DSymArgs b, const MU4* __restrict__ mu4,
+                                                       R* __restrict__ fwd, R* __restrict__ rev) {
   constexpr int TB = W * TS;
-  __shared__ SymTarget<R> tl[W][TS];
+  constexpr bool kAbs = sizeof(POS) == 8;
+  __shared__ SymTarget<R, POS> tl[W][TS];
   __shared__ R red[2][W][3][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int4 it  = b.items[blockIdx.x];
   const int I = it.x, kb = it.w;
-  const long long s0 = it.y, s1 = it.z;
-  const bool diag = s0 == (long long)I * TB;  // the tile's own sites (uniform over the block)
+  const int s0 = it.y, s1 = it.z;
+  const bool diag = s0 == I * TB;  // the tile's own sites (uniform over the block)
   const int t0    = I * TB + wv * TS;
   const int T     = max(0, min(TS, b.n - t0));
-  constexpr R kFar = sizeof(R) == 4 ? R(1.0e4) : R(1.0e8);
-  SymTarget<R>* tg = tl[wv];
+  constexpr POS kFar = POS(kAbs ? 1.0e8 : 1.0e4);
+  SymTarget<R, POS>* tg = tl[wv];
   if (lane < T) {
-    const TREC tr = trec[t0 + lane];
-    const MU4 mt  = mu4[t0 + lane];
-    tg[lane].p    = SymVec4<R>{(R)tr.x, (R)tr.y, (R)tr.z, (R)tr.w};
-    tg[lane].m    = SymVec4<R>{(R)mt.x, (R)mt.y, (R)mt.z, R(0)};
+    const double4 p = a.pos4[t0 + lane];
+    const MU4 mt    = mu4[t0 + lane];
+    tg[lane]        = SymTarget<R, POS>{(POS)(kAbs ? p.x : p.x - b.cx), (POS)(kAbs ? p.y : p.y - b.cy),
+                                        (POS)(kAbs ? p.z : p.z - b.cz), DAMP ? staged_di<R, B2>(a.damping, p.w) : R(0),
+                                        {(R)mt.x, (R)mt.y, (R)mt.z, R(0)}};
   }
   __syncthreads();
   R f[TS][3];
 #pragma unroll
   for (int t = 0; t < TS; ++t) f[t][0] = f[t][1] = f[t][2] = R(0);
-  __shared__ int2 mem[W][64];
-  unsigned ent;
-  const ItemSkips its(b.sk, t0, T, lane, mem[wv], ent);
-  const int partner = lane < its.n ? (int)(ent & kSkipSite) : -1;
+  __shared__ int mem[W][64];
+  const ItemSkips its(b.sk, t0, T, lane, mem[wv]);
   int buf = 0;
-  for (long long q0 = s0; q0 < s1; q0 += 64) {
-    const long long j = q0 + lane;
-    const bool act    = j < s1;
-    R xs = kFar, ys = kFar, zs = kFar, ss = R(0), mx = R(0), my = R(0), mz = R(0);
+  for (int q0 = s0; q0 < s1; q0 += 64) {
+    const int j    = q0 + lane;
+    const bool act = j < s1;
+    POS xs = kFar, ys = kFar, zs = kFar;
+    R ss = R(0), mx = R(0), my = R(0), mz = R(0);
     if (act) {
       const double4 pj = a.pos4[j];
       const MU4 mj     = mu4[j];
-      xs = sizeof(R) == 8 ? (R)pj.x : (R)(pj.x - b.cx);
-      ys = sizeof(R) == 8 ? (R)pj.y : (R)(pj.y - b.cy);
-      zs = sizeof(R) == 8 ? (R)pj.z : (R)(pj.z - b.cz);
+      xs = (POS)(kAbs ? pj.x : pj.x - b.cx);
+      ys = (POS)(kAbs ? pj.y : pj.y - b.cy);
+      zs = (POS)(kAbs ? pj.z : pj.z - b.cz);
       ss = (R)pj.w;
       mx = (R)mj.x;
       my = (R)mj.y;
       mz = (R)mj.z;
     }
-    unsigned skip = 0;  // targets that leave this source out
-    const unsigned long long in = __ballot(partner >= q0 && partner < q0 + 64);
-    if (in != 0 || its.n > 64) skip = its.template of<false>((int)j, in);
+    unsigned skip = its.template run<false>(q0, true) | its.template rest<false>(j);
     if (diag) {  // ordered pairs inside the tile
-      if (j >= t0 && j < t0 + T) skip |= 1u << (int)(j - t0);
+      if (j >= t0 && j < t0 + T) skip |= 1u << (j - t0);
 #pragma unroll
       for (int t = 0; t < TS; ++t) {
         if (t < T) {
-          const SymVec4<R> tp = tg[t].p;
-          const R dx = tp.x - xs, dy = tp.y - ys, dz = tp.z - zs;
+          const R dx = (R)(tg[t].x - xs), dy = (R)(tg[t].y - ys), dz = (R)(tg[t].z - zs);
           R c3, cf;
-          staged_geo<R, DAMP, B2, false, false>(dx, dy, dz, tp.w * ss, c3, cf, skip >> t & 1u);
+          staged_geo<R, DAMP, B2, false, false>(dx, dy, dz, tg[t].w * ss, c3, cf, keep_unless(skip, t));
           acc_m1(c3, cf, dx, dy, dz, mx, my, mz, f[t][0], f[t][1], f[t][2]);
         }
       }
@@ -367,19 +361,19 @@ __global__ __launch_bounds__(64 * W) void k_direct_sym(NearArgs a, DSymArgs b, c
     for (int t = 0; t < TS; ++t)
       if (t < T)
         sym_pair<R, DAMP, B2, false>(tg[t], xs, ys, zs, ss, mx, my, mz, f[t][0], f[t][1], f[t][2], rx, ry, rz,
-                                     skip >> t & 1u);
+                                     keep_unless(skip, t));
     red[buf][wv][0][lane] = rx;
     red[buf][wv][1][lane] = ry;
     red[buf][wv][2][lane] = rz;
     __syncthreads();  // (also orders this buffer's reads two stages back before it is rewritten)
     if (threadIdx.x < 3 * 64) {
       const int c = threadIdx.x >> 6, l = threadIdx.x & 63;
-      const long long jj = q0 + l;
+      const int jj = q0 + l;
       if (jj < s1) {
         R s = red[buf][0][c][l];
 #pragma unroll
         for (int w = 1; w < W; ++w) s += red[buf][w][c][l];
-        const int J = (int)(jj / TB), u = (int)(jj - (long long)J * TB);
+        const int J = jj / TB, u = jj - J * TB;
         rev[dsym_rev_block(J, I, TB) + c * TB + u] = s;
       }
     }

@@ -671,18 +671,18 @@ void build_pair_skips(System& S) {
 // Every entry of a cell's expanded near list in near-list order, one block per cell: the source site with
 // its class in the top bits. XC_OWN: the leaf's own sites. XC_PARTNER: sites of other leaves that the skip list of an
 // own site names. The others by the smallest Thole argument v = damping s_i s_j R_ij
-// over the leaf's own sites i (exact, FP64): XC_NEAR: v < 18, XC_MID: 18 <= v < 40, XC_FAR: v >= 40 (a small
-// margin above each bound). Undamped sites (s = 0) are XC_NEAR without the search, so are one-leaf
+// over the leaf's own sites i (exact, FP64): XC_NEAR: v < 18, XC_MID: 18 <= v < 25, XC_WIDE: 25 <= v < 40,
+// XC_FAR: v >= 40 (a small margin above each bound). Undamped sites (s = 0) are XC_NEAR without the search, so are one-leaf
 // (direct-summation) systems, all of whose sites are own, and cost O(n) here. The near
 // leaves are taken 256 at a time (prefix sums of their sizes in LDS), the entries 64 at a time by the
 // block's wavefronts, with the leaf's sites in LDS; a wavefront leaves the search once all its entries
 // are of class XC_NEAR. The ends of the classes (totals over the cell) go to ends.
-enum XClass : unsigned { XC_OWN = 0, XC_PARTNER, XC_NEAR, XC_MID, XC_FAR, XC_COUNT };
+enum XClass : unsigned { XC_OWN = 0, XC_PARTNER, XC_NEAR, XC_MID, XC_WIDE, XC_FAR, XC_COUNT };
 constexpr int kXclsShift = 29;
 constexpr unsigned kXclsSite = (1u << kXclsShift) - 1u;
-// ends of the classes XC_OWN, XC_PARTNER, XC_NEAR and XC_MID in the ordered list
+// ends of the classes XC_OWN, XC_PARTNER, XC_NEAR, XC_MID and XC_WIDE in the ordered list
 struct XEnds {
-  long long *own, *spec, *s32, *s64;
+  long long *own, *spec, *s32, *mid, *s64;
 };
 __global__ __launch_bounds__(256) void k_xclass(const int* __restrict__ off, const int* __restrict__ src,
                                                 const int* __restrict__ start, const int* __restrict__ count,
@@ -696,7 +696,7 @@ __global__ __launch_bounds__(256) void k_xclass(const int* __restrict__ off, con
   const int c = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const int o0 = off[c], o1 = off[c + 1];
   if (o0 == o1) {
-    if (tid == 0) ends.own[c] = ends.spec[c] = ends.s32[c] = ends.s64[c] = xoff[c];
+    if (tid == 0) ends.own[c] = ends.spec[c] = ends.s32[c] = ends.mid[c] = ends.s64[c] = xoff[c];
     return;
   }
   const int i0 = start[c], ni = count[c];
@@ -744,11 +744,14 @@ __global__ __launch_bounds__(256) void k_xclass(const int* __restrict__ off, con
           if ((i & 7) == 7 && __all(m < stop)) break;  // (of the lanes still searching)
         }
         const double v = damping * sj * sqrt(m);
-        cl = v < kFarClass32 * (1.0 + 1e-9) ? XC_NEAR : (v < kTholeCutoff * (1.0 + 1e-9) ? XC_MID : XC_FAR);
+        cl = v < kFarClass32 * (1.0 + 1e-9)      ? XC_NEAR
+             : v < kTholeCutoff32 * (1.0 + 1e-9) ? XC_MID
+             : v < kTholeCutoff * (1.0 + 1e-9)   ? XC_WIDE
+                                                 : XC_FAR;
       }
       if (q < total) ent[pos + q] = (unsigned)j | (cl << kXclsShift);
 #pragma unroll
-      for (unsigned k : {XC_OWN, XC_NEAR, XC_MID}) {
+      for (unsigned k : {XC_OWN, XC_NEAR, XC_MID, XC_WIDE}) {
         const int n = __popcll(__ballot(cl == k));
         if (lane == 0 && n) atomicAdd(&num[k], n);
       }
@@ -777,7 +780,8 @@ __global__ __launch_bounds__(256) void k_xclass(const int* __restrict__ off, con
     ends.own[c]  = e += num[XC_OWN];  // (a theta far above 1 can make a leaf far from itself: none)
     ends.spec[c] = e += num[XC_PARTNER];
     ends.s32[c]  = e += num[XC_NEAR];
-    ends.s64[c]  = e + num[XC_MID];
+    ends.mid[c]  = e += num[XC_MID];
+    ends.s64[c]  = e + num[XC_WIDE];
   }
 }
 
@@ -789,7 +793,7 @@ __global__ __launch_bounds__(256) void k_xfill(int ncells, const unsigned* __res
   if (c >= ncells) return;
   const unsigned long long below = (1ull << lane) - 1ull;
   const long long e0 = xoff[c], e1 = xoff[c + 1];
-  long long pos[XC_COUNT] = {e0, ends.own[c], ends.spec[c], ends.s32[c], ends.s64[c]};
+  long long pos[XC_COUNT] = {e0, ends.own[c], ends.spec[c], ends.s32[c], ends.mid[c], ends.s64[c]};
   for (long long e = e0; e < e1; e += 64) {
     const unsigned v = e + lane < e1 ? ent[e + lane] : 0xffffffffu;
     const unsigned k = v >> kXclsShift;
@@ -823,10 +827,11 @@ void build_near_expanded(System& S) {
   T.xspec.alloc(nc);
   T.xsplit[0].alloc(nc);
   T.xsplit[1].alloc(nc);
+  T.xsplit[2].alloc(nc);
   build_pair_skips(S);
   dbuf<long long> xown;
   xown.alloc(nc);
-  const XEnds ends{xown.p, T.xspec.p, T.xsplit[1].p, T.xsplit[0].p};
+  const XEnds ends{xown.p, T.xspec.p, T.xsplit[1].p, T.xsplit[2].p, T.xsplit[0].p};
   // (site indices below 2^29: a system of more sites has no room for its lists on the device)
   dbuf<unsigned> ent;
   ent.alloc(std::max<long long>(total, 1));

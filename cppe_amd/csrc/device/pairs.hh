@@ -4,19 +4,35 @@
 
 namespace cppe_dev {
 
+// v where keep has all bits set, zero where it has none (of any v, infinities included).
+__device__ __forceinline__ float kept(float v, int keep) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(int, v) & keep);
+}
+__device__ __forceinline__ double kept(double v, int keep) {
+  int2 b = __builtin_bit_cast(int2, v);
+  b.x &= keep;
+  b.y &= keep;
+  return __builtin_bit_cast(double, b);
+}
+// that mask from bit t of skip
+__device__ __forceinline__ int keep_unless(unsigned skip, int t) {
+  return __builtin_amdgcn_sbfe((int)~skip, t, 1);  // (shifts the compiler turns into a compare and a select)
+}
+
 // ---------------------------------------------------------------------------------------------
 // Pair kernels. d = r_target - r_source.
 // ---------------------------------------------------------------------------------------------
 // -T2 mu with Thole damping: fE mu / R^3 - 3 fT (d.mu) d / R^5  (P2P<1,3>, field_m1.cc:127-193),
 // split into the pair's geometry (c3 = fE / R^3, cf = 3 fT / R^5) and the accumulation of one
 // dipole, so that several dipole vectors can share one geometry evaluation.
-// SELF0: a zero displacement (a site with itself) contributes exactly zero. skip: so does this pair.
+// SELF0: a zero displacement (a site with itself) contributes exactly zero. keep: all bits set, or none: so does
+// this pair then, whatever its displacement (1/R is masked: one and-operation for 32 bits).
 template <bool DAMP, bool SELF0 = false>
 __device__ __forceinline__ void geo_m1_f64(double dx, double dy, double dz, double a, double& c3, double& cf,
-                                           bool skip = false) {
+                                           int keep = -1) {
   const double r2   = dx * dx + dy * dy + dz * dz;
   const double rsq  = rsqrt_f64(r2);
-  const double rinv = skip || (SELF0 && !(r2 > 0.0)) ? 0.0 : rsq;
+  const double rinv = SELF0 ? (r2 > 0.0 ? rsq : 0.0) : kept(rsq, keep);
   const double ri2  = rinv * rinv;
   const double ri3  = rinv * ri2;
   double fE = 1.0, fT = 1.0;
@@ -30,10 +46,10 @@ __device__ __forceinline__ void geo_m1_f64(double dx, double dy, double dz, doub
 
 template <bool DAMP, bool SELF0 = false>
 __device__ __forceinline__ void geo_m1_f32(float dx, float dy, float dz, float a, float& c3, float& cf,
-                                           bool skip = false) {
+                                           int keep = -1) {
   const float r2   = dx * dx + dy * dy + dz * dz;
   const float rsq  = rsqrt_f32(r2);
-  const float rinv = skip || (SELF0 && !(r2 > 0.0f)) ? 0.0f : rsq;
+  const float rinv = SELF0 ? (r2 > 0.0f ? rsq : 0.0f) : kept(rsq, keep);
   const float ri2  = rinv * rinv;
   const float ri3  = rinv * ri2;
   float fE = 1.0f, fT = 1.0f;
@@ -50,18 +66,17 @@ __device__ __forceinline__ void geo_m1_f32(float dx, float dy, float dz, float a
 // base-2 units (v = u2 ln 2) and e^-v = 2^-u2 comes straight from v_exp_f32. With v = u2 ln2
 //   f_E = 1 - (1 + ln2 u2 + (ln2)^2/2 u2^2) 2^-u2,   f_T = f_E - (ln2)^3/6 u2^3 2^-u2.
 // SELF0: a zero displacement (the site itself) contributes exactly zero: 1/R is clamped to 2^40, so
-// R = 0, u2 = 0, 2^-u2 = 1 and f_E = f_T = 0 exactly (this needs a2 finite, i.e. damped sites). A skipped
-// pair has 1/R = 0 in place of it.
+// R = 0, u2 = 0, 2^-u2 = 1 and f_E = f_T = 0 exactly (this needs a2 finite, i.e. damped sites). keep as above.
 // Large u2 (undamped in effect) gives 2^-u2 = 0 and f_E = f_T = 1.
 template <bool SELF0>
 __device__ __forceinline__ void geo_m1_f32_b2(float dx, float dy, float dz, float a2, float& c3, float& cf,
-                                              bool skip = false) {
+                                              int keep = -1) {
   constexpr float kC1 = 0.693147180559945309f;   // ln 2
   constexpr float kC2 = 0.240226506959100712f;   // (ln 2)^2 / 2
   constexpr float kC3 = 0.0555041086648215800f;  // (ln 2)^3 / 6
   const float r2   = dx * dx + dy * dy + dz * dz;
   const float rsq  = rsqrt_f32(r2);
-  const float rinv = skip ? 0.0f : SELF0 ? __builtin_fminf(rsq, 1099511627776.0f) /* 2^40 */ : rsq;
+  const float rinv = SELF0 ? __builtin_fminf(rsq, 1099511627776.0f) /* 2^40 */ : kept(rsq, keep);
   const float ri2  = rinv * rinv;
   const float ri3  = ri2 * rinv;
   const float u    = a2 * (r2 * rinv);

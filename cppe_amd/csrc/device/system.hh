@@ -62,11 +62,11 @@ struct Octree {
   dbuf<int> xsrc;              // source sites (device order)
   // Each leaf's expanded list begins with its own sites and the sites that their skip lists name in other leaves (up
   // to xspec: the only entries that can be a target itself or a pair left out); the rest is ordered by the
-  // smallest Thole argument v of each source over the leaf's targets: v_min < 18, then 18 <= v_min < 40,
-  // then v_min >= 40 (each class in near-list order).
-  // xsplit[1] (FP32) / xsplit[0] (FP64): offset of the first source that takes the undamped pair
-  // in that precision for every target of the leaf (kFarClass32, kTholeCutoff).
-  dbuf<long long> xspec, xsplit[2];
+  // smallest Thole argument v of each source over the leaf's targets: v_min < 18, then < 25, then < 40, then the
+  // rest (each class in near-list order). Offset of the first source that takes the undamped pair for every target
+  // of the leaf: xsplit[0] FP64 (kTholeCutoff), xsplit[1] FP32 (kFarClass32), xsplit[2] FP32 of untuned systems
+  // (kTholeCutoff32, from where on FP32 pairs everywhere are undamped).
+  dbuf<long long> xspec, xsplit[3];
   double xdamp = 0.0;  // damping factor of the classification (valid for kernels with damping >= xdamp)
   SymLists sym[2][5];  // symmetric near field (FP64, FP32) with chunks of 4, 6, 8, 12, 16 targets (sym_slot)
   int near_symmetric = -1;  // near_lists_symmetric's answer (-1: not asked yet)
