@@ -1,11 +1,12 @@
 // Device memory of a system and transfers of pageable host memory.
 //
 // What bounds a short run is the host: hipMalloc and hipFree of blocks of a MiB and more take 30 to 330 us
-// each (smaller ones 1 us, from the runtime's own pool), a system makes some 90, and the runtime copies
+// each (smaller ones 1 us, from the runtime's own pool, but 280 us where that pool has just been emptied by
+// the last system's end and is mapped again), a system makes some 90, and the runtime copies
 // pageable arrays of 64 KiB to 3 MiB at 2.9 GB/s. So blocks of kArenaMin and more come from chunks a system
 // keeps (DeviceArena), chunks outlive it in a bounded pool, and such arrays go through pinned slots: the static
-// fields and energies of 120,000 sites, system included, took 15.2 ms and now 5.6, a geometry step of 24,000
-// sites 15.9 and 9.8, the loss and gradient of 63,001 samples (arena alone) 1.18 and 1.02.
+// fields and energies of 120,000 sites, system included, took 15.2 ms and now 5.4, a geometry step of 24,000
+// sites 15.9 and 8.4, the loss and gradient of 63,001 samples (arena alone) 1.18 and 1.02.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -26,7 +27,9 @@ void* device_malloc(size_t bytes);
 // taken again at once, as what used it comes before in that order. Used by one thread at a time, as its owner.
 class DeviceArena {
  public:
-  static constexpr size_t kArenaMin = size_t(1) << 19;  // below, the runtime's own pool is as fast
+  // Smaller blocks come from the runtime's own pool. With 512 KiB here a geometry step of 24,000 sites mapped
+  // that pool anew once or twice in each pass: 8.9 to 9.7 ms, 8.3 to 8.5 with 64 (and with 16).
+  static constexpr size_t kArenaMin = size_t(1) << 16;
   explicit DeviceArena(hipStream_t st = nullptr) : stream(st) {}
   DeviceArena(const DeviceArena&) = delete;
   DeviceArena& operator=(const DeviceArena&) = delete;

@@ -11,8 +11,8 @@ namespace cppe_dev {
 
 // ---- chunks ----------------------------------------------------------------------------------
 // A chunk is at least kChunkMin and grows with what the arena holds already, so a system of any size has
-// few; a request above kChunkPooled has a chunk of its own, which goes back to the device when it is free.
-constexpr size_t kChunkMin    = size_t(8) << 20;
+// few and a small one (some ten blocks of 64 KiB and more at 1,000 sites) holds little; a request above kChunkPooled has a chunk of its own, which goes back to the device when it is free.
+constexpr size_t kChunkMin    = size_t(2) << 20;
 constexpr size_t kChunkPooled = size_t(256) << 20;
 constexpr size_t kPoolBytes   = size_t(512) << 20;  // most the pool holds over all devices
 constexpr auto kPoolAge       = std::chrono::seconds(10);
