@@ -1,11 +1,17 @@
 // Chunk pool, arenas and pinned staging (memory.hh).
 #include "memory.hh"
 
+#include <unistd.h>
+
 #include <algorithm>
 #include <chrono>
+#include <condition_variable>
+#include <cstdlib>
 #include <cstring>
 #include <memory>
 #include <mutex>
+#include <system_error>
+#include <thread>
 
 namespace cppe_dev {
 
@@ -20,10 +26,18 @@ constexpr size_t kAlign       = 256;
 
 using Clock = std::chrono::steady_clock;
 
-// Free chunks for any thread; one not asked for within kPoolAge goes back to the device with the next
-// call, the oldest ones when the bound is passed, all when an allocation fails.
+// Free chunks for any thread; one not asked for within kPoolAge goes back to the device, the oldest ones when
+// the bound is passed, all when an allocation fails. What keeps the time is a thread that lives as long as there
+// are free chunks: a program that has ended its work leaves nothing on a device that others use.
 class ChunkPool {
  public:
+  ChunkPool() : pid(getpid()) {
+    std::atexit([] { instance().stop_timer(); });  // (registered after the runtime's own, so it runs before)
+  }
+  static ChunkPool& instance() {
+    static ChunkPool* p = new ChunkPool;  // never destroyed: systems may go after static destructors have run
+    return *p;
+  }
   // a chunk of at least want bytes on the device (its size in size), or none
   void* take(size_t want, int dev, size_t& size) {
     std::vector<void*> old;
@@ -54,6 +68,7 @@ class ChunkPool {
       free.push_back({p, size, dev, Clock::now()});
       held += size;
       while (held > kPoolBytes) pop_front(old);
+      start_timer();
     }
     drop(old);
   }
@@ -85,16 +100,50 @@ class ChunkPool {
   static void drop(const std::vector<void*>& old) {
     for (void* p : old) (void)hipFree(p);
   }
+  // (m held) A thread that has ended has let go of m for good; a forked child has no such thread, and no device.
+  void start_timer() {
+    if (timed || stopped || free.empty() || getpid() != pid) return;
+    if (timer.joinable()) timer.join();
+    try {
+      timer = std::thread([this] { run_timer(); });
+      timed = true;
+    } catch (const std::system_error&) {  // no thread to be had: chunks age with the next calls
+    }
+  }
+  void run_timer() {
+    // hipFree here must not end a capture that another thread has begun
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    std::unique_lock<std::mutex> lock(m);
+    while (!stopped && !free.empty()) {
+      wake.wait_until(lock, free.front().since + kPoolAge + std::chrono::milliseconds(1));
+      std::vector<void*> old;
+      if (!stopped) expire(old);
+      lock.unlock();
+      drop(old);
+      lock.lock();
+    }
+    timed = false;
+  }
+  void stop_timer() {
+    if (getpid() != pid) return;
+    {
+      std::lock_guard<std::mutex> lock(m);
+      stopped = true;
+    }
+    wake.notify_all();
+    if (timer.joinable()) timer.join();
+  }
   std::mutex m;
+  std::condition_variable wake;
+  std::thread timer;
+  const pid_t pid;
+  bool timed = false, stopped = false;
   std::vector<Entry> free;  // oldest first
   size_t held = 0;
 };
 
-// (never destroyed: systems may go after static destructors have run, and the device frees the rest)
-static ChunkPool& pool() {
-  static ChunkPool* p = new ChunkPool;
-  return *p;
-}
+static ChunkPool& pool() { return ChunkPool::instance(); }
 
 void* device_malloc(size_t bytes) {
   void* p      = nullptr;
