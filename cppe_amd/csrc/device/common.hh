@@ -11,6 +11,10 @@ namespace cppe_dev {
 struct hip_error : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
+// no device memory left for an allocation
+struct out_of_memory : hip_error {
+  using hip_error::hip_error;
+};
 
 #define CPPE_HIP_CHECK(expr)                                                                 \
   do {                                                                                       \

@@ -95,8 +95,84 @@ static FmmState& state(System& S) {
   return *S.fmm;
 }
 
+static void drop_symmetric(System& S, int prec) {
+  FmmState& F = *S.fmm;
+  for (SymLists& Y : S.tree.sym[prec]) {
+    Y.ts = 0;
+    Y.items.release();
+    Y.uoff.release();
+    Y.usplit.release();
+    Y.rev_off.release();
+    Y.usrc.release();
+    Y.nin.release();
+    Y.udst.release();
+  }
+  if (prec) {
+    F.dfwd32.release();
+    F.drev32.release();
+    F.rev32.release();
+  } else {
+    F.dfwd64.release();
+    F.drev64.release();
+    F.rev64.release();
+  }
+}
+
+// Lists and buffers of the near-field form that precision prec takes. Untuned systems take their forms for speed: without
+// memory for the reverse blocks of the symmetric one they take lanes as sources, without memory for its expanded
+// lists the thread-per-target form, which has neither. A chosen form keeps the error.
+static void ensure_near_form(System& S, int prec) {
+  FmmState& F = *S.fmm;
+  Octree& T   = S.tree;
+  for (;;) {
+    const int v = F.tune.near_variant[prec];
+    if (F.near_ready[prec] == v) return;
+    try {
+      if (near_sym_variant(v)) {
+        if (one_leaf_system(S))
+          ensure_dsym(S, prec, kSymTs[prec][v - 9]);
+        else
+          ensure_sym(S, prec, kSymTs[prec][v - 9], S.opts.damping);
+      } else if (v == 3 || v >= 5) {
+        build_near_expanded(S);
+        if (near_lanes_variant(v))
+          ensure_near_chunks(S, near_lanes_ts(v, prec, 1));
+        else if (v >= 5)
+          ensure_near_items(S, v - 5);
+      }
+      if (v == 1 || v == 3) ensure_near_items(S, 0);
+      F.near_ready[prec] = v;
+      return;
+    } catch (const out_of_memory&) {
+      if (!F.tune.own_displacements || v == 0) throw;
+      if (near_sym_variant(v)) drop_symmetric(S, prec);
+      if (T.nx < 0) {
+        T.xoff.release();
+        T.xsrc.release();
+      }
+      F.tune.near_variant[prec] = !near_sym_variant(v) ? 0 : one_leaf_system(S) || prec ? 8 : 7;
+      F.tune.near_block[prec]   = 256;
+    }
+  }
+}
+
+// Lists of the lanes form with chunks of ts targets, for launches that take it whatever symmetric form the system has;
+// without memory for them as in ensure_near_form (right-hand sides one at a time then).
+static void ensure_lanes(System& S, int prec, int ts) {
+  FmmState& F = *S.fmm;
+  try {
+    build_near_expanded(S);
+    ensure_near_chunks(S, ts);
+  } catch (const out_of_memory&) {
+    if (!F.tune.own_displacements) throw;
+    F.tune.near_variant[prec] = 0;
+    F.tune.near_block[prec]   = 256;
+  }
+}
+
 void apply_b_fmm(System& S, const double* x, double* out, bool fp32) {
   state(S);
+  ensure_near_form(S, fp32 ? 1 : 0);
 #define CALL(P) fmm_apply_b_t<P>(S, x, out, fp32)
   CPPE_FMM_DISPATCH(CALL)
 #undef CALL
@@ -141,12 +217,8 @@ void fmm_reserve_multi(System& S, bool mixed) {
   }
   ensure_pos4(S);
   build_pair_skips(S);
-  for (int prec = 0; prec <= (mixed ? 1 : 0); ++prec) {
-    const int v = F.tune.near_variant[prec];
-    if (v < 5) continue;
-    build_near_expanded(S);
-    ensure_near_chunks(S, near_lanes_ts(8, prec, kMultiRhs));
-  }
+  for (int prec = 0; prec <= (mixed ? 1 : 0); ++prec)
+    if (F.tune.near_variant[prec] >= 5) ensure_lanes(S, prec, near_lanes_ts(8, prec, kMultiRhs));
   CPPE_HIP_CHECK(hipStreamSynchronize(S.stream));
 }
 
@@ -163,6 +235,8 @@ void fmm_field(System& S, int m, const double* src, double* F, double damping, b
   (void)fp32;
   FmmState& st = state(S);
   if (m == 1) {
+    const int v = st.tune.near_variant[0];
+    if (v >= 7) ensure_lanes(S, 0, near_lanes_ts(v == 7 ? 7 : 8, 0, 1));
 #define CALL(P) fmm_field1_t<P>(S, src, F, damping)
     CPPE_FMM_DISPATCH(CALL)
 #undef CALL
@@ -293,22 +367,10 @@ void fmm_reserve(System& S, bool mixed, int nrhs) {
     ensure_m2l_rec(S, S.stream);  // the synchronisation below orders it before any stream's M2L
   }
   for (int prec = 0; prec < np && !grouped; ++prec) {
+    ensure_near_form(S, prec);
     const int v = F.tune.near_variant[prec];
-    if (v == 1 || v == 3) ensure_near_items(S, 0);
     if (prec == 1 && (v == 1 || v == 4)) ensure_posf4(S);
     if (v == 4) ensure_clusters(S);
-    if (near_sym_variant(v)) {
-      if (one_leaf_system(S))
-        ensure_dsym(S, prec, kSymTs[prec][v - 9]);
-      else
-        ensure_sym(S, prec, kSymTs[prec][v - 9], S.opts.damping);
-    } else if (v == 3 || v >= 5) {
-      build_near_expanded(S);
-      if (near_lanes_variant(v))
-        ensure_near_chunks(S, near_lanes_ts(v, prec, 1));
-      else if (v >= 5)
-        ensure_near_items(S, v - 5);
-    }
   }
   CPPE_HIP_CHECK(hipStreamSynchronize(S.stream));
   for (int prec = 0; prec < np && !grouped; ++prec) F.reserved_for[prec] = F.tune.near_variant[prec];

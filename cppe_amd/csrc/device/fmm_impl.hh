@@ -84,6 +84,7 @@ struct FmmState {
   dbuf<double> Mc, Lc;    // combined kind (static fields, m = 0 / 2)
   dbuf<double> src10;     // staging of combined sources
   dbuf<double4> pos4;     // near-field source records: x, y, z, alpha_iso^(-1/6)
+  int near_ready[2]   = {-1, -1};  // near variants (FP64, FP32) whose lists and buffers are there (ensure_near_form)
   int reserved_for[2] = {-1, -1};  // near variants (FP64, FP32) fmm_reserve last prepared for
   dbuf<double4> mu4;      // near-field dipole records (FP64 form)
   dbuf<float4> mu4f;      // near-field dipole records (FP32 form)

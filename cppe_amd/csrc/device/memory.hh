@@ -20,7 +20,7 @@
 
 namespace cppe_dev {
 
-// hipMalloc that empties the chunk pool and tries again before it gives up.
+// hipMalloc that empties the chunk pool and tries again before it gives up (throws out_of_memory).
 void* device_malloc(size_t bytes);
 
 // Blocks of one owner whose work is all ordered on one stream (others join it): a block given back may be

@@ -4,8 +4,10 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <condition_variable>
+#include <cstdint>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
@@ -14,6 +16,12 @@
 #include <thread>
 
 namespace cppe_dev {
+
+// Largest allocation that succeeds: a bound for tests of what happens when there is no memory.
+static std::atomic<size_t> g_most{SIZE_MAX};
+extern "C" void cppe_hip_test_largest_allocation(long long bytes) {
+  g_most = bytes > 0 ? (size_t)bytes : SIZE_MAX;
+}
 
 // ---- chunks ----------------------------------------------------------------------------------
 // A chunk is at least kChunkMin and grows with what the arena holds already, so a system of any size has
@@ -145,7 +153,9 @@ class ChunkPool {
 
 static ChunkPool& pool() { return ChunkPool::instance(); }
 
-void* device_malloc(size_t bytes) {
+// null where the device has no room
+static void* try_malloc(size_t bytes) {
+  if (bytes > g_most) return nullptr;
   void* p      = nullptr;
   hipError_t e = hipMalloc(&p, bytes);
   if (e == hipErrorOutOfMemory) {
@@ -153,7 +163,17 @@ void* device_malloc(size_t bytes) {
     pool().clear();
     e = hipMalloc(&p, bytes);
   }
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
   CPPE_HIP_CHECK(e);
+  return p;
+}
+
+void* device_malloc(size_t bytes) {
+  void* p = try_malloc(bytes);
+  if (!p) throw out_of_memory("out of device memory: " + std::to_string(bytes) + " bytes");
   return p;
 }
 
@@ -165,6 +185,7 @@ static size_t rounded(size_t bytes) { return (bytes + kAlign - 1) / kAlign * kAl
 
 void* DeviceArena::take(size_t bytes) {
   const size_t need = rounded(bytes);
+  if (bytes > g_most) throw out_of_memory("out of device memory: " + std::to_string(bytes) + " bytes");
   // the smallest hole that fits
   Chunk* at = nullptr;
   std::map<size_t, size_t>::iterator hole;
@@ -182,10 +203,12 @@ void* DeviceArena::take(size_t bytes) {
     if (need <= kChunkPooled) {
       size = kChunkMin;
       while (size < need || (size < total && size < kChunkPooled)) size *= 2;
+      if (size > g_most) size = need;
       p = pool().take(size, dev, size);
     }
     chunks.reserve(chunks.size() + 1);
-    if (!p) p = device_malloc(size);
+    if (!p && size > need) p = try_malloc(size);
+    if (!p) p = device_malloc(size = need);  // (no room to grow: what is asked for alone)
     chunks.push_back({static_cast<char*>(p), size, 0, dev, {}});
     total += size;
     at = &chunks.back();
