@@ -61,6 +61,9 @@ struct FmmState {
   hipStream_t far_stream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   ~FmmState() {
+    // (an apply that ended with an error between fork and join leaves work here that no other stream waits for, on
+    // blocks that serve another system next)
+    if (far_stream) (void)hipStreamSynchronize(far_stream);
     if (ev_fork) (void)hipEventDestroy(ev_fork);
     if (ev_join) (void)hipEventDestroy(ev_join);
     if (far_stream) (void)hipStreamDestroy(far_stream);
