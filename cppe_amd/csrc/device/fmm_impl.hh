@@ -68,9 +68,9 @@ struct FmmState {
     if (ev_join) (void)hipEventDestroy(ev_join);
     if (far_stream) (void)hipStreamDestroy(far_stream);
   }
-  // work items (leaf, first target) of the leaf-chunk near kernels, for chunks of 64, 32, 16, 8 targets
-  dbuf<int2> near_items[4];
-  int n_items[4] = {0, 0, 0, 0};
+  // work items (leaf, first target) of the leaf-chunk near kernels, for chunks of 64, 32, 8 targets
+  dbuf<int2> near_items[3];
+  int n_items[3] = {0, 0, 0};
   // chunks of the lanes-as-sources near kernel: (leaf, first site, sites, 0), at most 16, 8, 4 targets
   dbuf<int4> near_chunks[3];
   int n_chunks[3] = {0, 0, 0};
@@ -1685,12 +1685,13 @@ inline void ensure_pos4(System& S) {
 }
 
 // Work items of the leaf-chunk near kernels: (leaf, first target) per chunk of at most C targets of
-// every leaf (C = 64 >> ci, ci = 0..3). Returns the item count.
+// every leaf, C = 64, 32 and kStaticTs for ci = 0, 1, 2. Returns the item count.
+constexpr int near_items_size(int ci) { return ci < 2 ? 64 >> ci : kStaticTs; }
 inline int ensure_near_items(System& S, int ci = 0) {
   FmmState& F     = *S.fmm;
   const Octree& T = S.tree;
   if (F.near_items[ci].p && F.n_items[ci] > 0) return F.n_items[ci];
-  const int C = 64 >> ci;
+  const int C = near_items_size(ci);
   const std::vector<int>&ids = T.h_leaf_ids, &cnt = T.h_count;
   std::vector<int2> items;
   items.reserve(T.nleaves);
@@ -2322,15 +2323,15 @@ void fmm_static_t(System& S, const double* src10, double* out, double damping) {
   const bool has_far = S.tree.n_m2l > 0;  // no cell pair: every local expansion is zero
   if (has_far) fmm_far_pass<KIND_MC, P, double>(S, src10, F.Mc.p, F.Lc.p, S.stream);
   static_records(S, 3, src10);
-  const int ni    = ensure_near_items(S, 3);  // chunks of kStaticTs targets
+  const int ni    = ensure_near_items(S, 2);  // chunks of kStaticTs targets
   P2PArgs a       = make_p2p_args(S, src10, damping, out);
   const auto* rec = reinterpret_cast<const StaticRec*>(S.static_rec.p);
   const dim3 g(ceil_div(ni, 4)), b(256);
   const double* L = has_far ? F.Lc.p : nullptr;
   if (damping > 0.0)
-    hipLaunchKernelGGL((k_fmm_near_static<P, true>), g, b, 0, S.stream, a, F.near_items[3].p, ni, rec, L);
+    hipLaunchKernelGGL((k_fmm_near_static<P, true>), g, b, 0, S.stream, a, F.near_items[2].p, ni, rec, L);
   else
-    hipLaunchKernelGGL((k_fmm_near_static<P, false>), g, b, 0, S.stream, a, F.near_items[3].p, ni, rec, L);
+    hipLaunchKernelGGL((k_fmm_near_static<P, false>), g, b, 0, S.stream, a, F.near_items[2].p, ni, rec, L);
 }
 
 #define CPPE_INSTANTIATE_FMM(P)                                                          \
