@@ -108,8 +108,9 @@ struct dbuf {
   DeviceArena* arena = nullptr;  // whose block this is (none: hipMalloc's)
 };
 
-// Copies on a stream from and to host memory of any kind. to_device returns once src may change, to_host
-// once dst holds the data.
+// Copies on a stream from and to host memory of any kind. to_device returns once pageable src may change; pinned src
+// must stay as it is until the stream has passed the copy (every entry point waits for its stream before it returns).
+// to_host returns once dst holds the data.
 void to_device(void* dst, const void* src, size_t bytes, hipStream_t st);
 void to_host(void* dst, const void* src, size_t bytes, hipStream_t st);
 
