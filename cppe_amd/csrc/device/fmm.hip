@@ -56,20 +56,15 @@ static FmmTune default_tune(System& S) {
   // Trees: lanes as sources. FP32: chunks of 8 targets (16 positions of 64 bits do not fit the scalar registers).
   t.near_variant[1] = 8;
   t.near_block[1]   = 256;
-  // FP64: chunks of 4; the symmetric form for the plain form's solves of some systems, where sharing a
-  // pair's geometry outweighs the reverse blocks (a mixed solve runs one or two FP64 applies, which would not pay for its
-  // lists): three values for each unordered pair of a site and an item, of kSymTs targets at most. It needs near lists
-  // that are symmetric, which those of a theta near 1 are not.
-  long long items = 0;
-  int most        = 0;
-  for (int c : T.h_leaf_ids) {
-    items += ceil_div(T.h_count[c], kSymTs[0][0]);
-    most = std::max(most, T.h_count[c]);
-  }
-  const double rev = 1.5 * (double)T.p2p_site_pairs * (double)items / S.n * sizeof(double);
-  const bool sym   = S.opts.precision == CPPE_HIP_PREC_FP64 && S.has_alpha && S.n >= kSymTreeSites &&
-                   rev <= kSymRevBytes && S.n >= (long long)kSymLeafLeast * T.nleaves &&
-                   S.n < (long long)kSymLeafMost * T.nleaves && most <= kSymLeafMax && near_lists_symmetric(S);
+  // FP64: chunks of 4; the symmetric form for the plain form's solves of larger systems with small
+  // leaves, where sharing a pair's geometry outweighs the reverse blocks (a mixed solve runs one or
+  // two FP64 applies, which would not pay for its lists). Its reverse slots are 32-bit indices: at
+  // most 3 values per site pair of different leaves, each unordered pair once. It needs near lists that
+  // are symmetric, which those of a theta near 1 are not.
+  const bool plain  = S.opts.precision == CPPE_HIP_PREC_FP64;
+  const bool fits   = 1.5 * (double)T.p2p_site_pairs < 2147483647.0;
+  const bool sym    = plain && fits && S.n >= kSymTreeSites && S.n < (long long)kSymLeafSites * T.nleaves &&
+                   S.has_alpha && near_lists_symmetric(S);
   t.near_variant[0] = sym ? 9 : 7;
   t.near_block[0]   = sym ? 128 : 256;
   t.m2l_group[0] = t.m2l_group[1] = T.ncells < kM2lWideCells ? 64 : 16;

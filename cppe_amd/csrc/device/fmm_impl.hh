@@ -1896,16 +1896,11 @@ constexpr double kDSymDefaultBytes = 4.0e9;
 // Sites from which an untuned direct-summation system takes FP32 chunks of 12 targets instead of 8
 // (apply at 9,000 sites 102 us either way, at 24,000 397 against 421 us, at 60,000 2.05 against 2.17 ms).
 constexpr int kDSym32Wide = 16384;
-// Where an untuned plain-form tree takes the symmetric near field (FP64 solves, lanes as sources / symmetric):
-// * its reverse blocks (estimated) stay within about the 256 MB last-level cache: 8.4 / 7.9 ms with 250 MB at 60,000
-//   sites, 10.1 / 9.7 with 285 at 66,000, 9.9 / 10.0 with 301 at 69,000, 11.7 / 12.0 at 75,000, 31.5 / 33.7 at 150,000;
-// * from 49,152 sites on: below, the items of a coarse leaf, whose upper lists are long, outlast the others (42,000 sites,
-//   ncrit 64 and leaves of 13: 6.3 / 8.3; ncrit 48 and leaves of 11: 5.8 / 5.1; 33,000: 5.1 / 6.3; 51,000: 7.0 / 6.2);
-// * leaves of 8 to 18 sites on average: 8.44 / 8.40 with 3.4 at 60,000 sites, 14.3 / 17.3 with 4 at 120,000;
-// * none above 64, again for the coarse ones: 8.5 / 10.4 with one of 95 at 54,000 sites, 9.0 / 10.0 with one of 79 at 60,000.
-constexpr int kSymTreeSites  = 49152;
-constexpr double kSymRevBytes = 288.0e6;
-constexpr int kSymLeafLeast = 8, kSymLeafMost = 18, kSymLeafMax = 64;
+// Sites and mean leaf size for which an untuned plain-form tree takes the symmetric near field: FP64
+// solves with it / with lanes as sources took 3.3 / 2.6 ms at 12,000 sites (23 a leaf), 7.7 / 8.2 at 60,000 (15
+// a leaf), 24.0 / 23.9 at 120,000 (29 a leaf) and 34.4 / 35.6 at 300,000 (10 a leaf).
+constexpr int kSymTreeSites = 49152;
+constexpr int kSymLeafSites = 18;
 // Cells from which an untuned system's M2L takes 16 lanes per target cell instead of 64: with fewer
 // cells 16 lanes leave SIMDs idle (FP64 at 24,000 sites / 585 cells 18 us with 64 lanes, 45 with 16; at
 // 60,000 sites / 4,700 cells 58 and 69; at 300,000 sites / 37,000 cells 464 and 429).
