@@ -1896,9 +1896,22 @@ constexpr double kDSymDefaultBytes = 4.0e9;
 // Sites from which an untuned direct-summation system takes FP32 chunks of 12 targets instead of 8
 // (apply at 9,000 sites 102 us either way, at 24,000 397 against 421 us, at 60,000 2.05 against 2.17 ms).
 constexpr int kDSym32Wide = 16384;
-// Sites and mean leaf size for which an untuned plain-form tree takes the symmetric near field: FP64
-// solves with it / with lanes as sources took 3.3 / 2.6 ms at 12,000 sites (23 a leaf), 7.7 / 8.2 at 60,000 (15
-// a leaf), 24.0 / 23.9 at 120,000 (29 a leaf) and 34.4 / 35.6 at 300,000 (10 a leaf).
+// Sites and mean leaf size for which an untuned plain-form tree takes the symmetric near field. FP64 solves of water
+// boxes with ncrit 16 to 64, lanes as sources / symmetric: a new system with its lists and first solve, and a
+// further solve of the same system (ms):
+//   sites   a leaf   new           again            sites   a leaf   new           again
+//   12,000  23                      2.6 /  3.3      69,000  17       21.1 / 21.3   10.3 / 10.4
+//   36,000  8.8 (at most 21)        4.7 /  4.2      75,000  18.5     24.3 / 24.6   11.8 / 12.2
+//   36,000  8.9 (at most 47)        4.7 /  5.5      99,000  3.4      32.4 / 33.0   13.7 / 16.7
+//   42,000  11.2                    5.8 /  5.1     120,000  7.6      36.5 / 34.8   17.2 / 17.5
+//   42,000  12.8 (at most 63)       6.3 /  8.3     120,000  29       42.4 / 42.5   23.6 / 25.0
+//   51,000  12.6     15.9 / 14.6    7.2 /  6.6     180,000  6.2      46.7 / 46.7   19.3 / 19.9
+//   60,000  3.4      21.7 / 19.5    8.8 /  8.7     240,000  15       83.4 / 79.9   47.1 / 47.7
+//   60,000  15       19.5 / 18.4    9.0 /  8.2     300,000  10       79.1 / 76.2   39.5 / 38.4
+// Below the bound on the sites a coarse leaf, whose upper lists are long, outlasts the other items in some boxes; from
+// it on this is rarer (a leaf of 95 at 54,000 sites: 8.5 / 10.4 again). Above the bound on the leaves the
+// reverse blocks cost more than they save. The other form's expanded lists cost a new system 0.5 to 5 ms more: large
+// systems of small leaves stay with the symmetric form although it gains nothing in further solves.
 constexpr int kSymTreeSites = 49152;
 constexpr int kSymLeafSites = 18;
 // Cells from which an untuned system's M2L takes 16 lanes per target cell instead of 64: with fewer
