@@ -25,7 +25,8 @@ extern "C" void cppe_hip_test_largest_allocation(long long bytes) {
 
 // ---- chunks ----------------------------------------------------------------------------------
 // A chunk is at least kChunkMin and grows with what the arena holds already, so a system of any size has
-// few and a small one (some ten blocks of 64 KiB and more at 1,000 sites) holds little; a request above kChunkPooled has a chunk of its own, which goes back to the device when it is free.
+// few and a small one (some ten blocks of 64 KiB and more at 1,000 sites) holds little; a request above
+// kChunkPooled has a chunk of its own, which goes back to the device when it is free.
 constexpr size_t kChunkMin    = size_t(2) << 20;
 constexpr size_t kChunkPooled = size_t(256) << 20;
 constexpr size_t kPoolBytes   = size_t(512) << 20;  // most the pool holds over all devices
